@@ -27,10 +27,23 @@
 //    to the lane (mod 32), then O^T(128 x 32) += V^T . P^T with 16 MFMAs, P
 //    taken straight from the S^T accumulators, rounded to the storage type
 //    (the reference's Triton kernel rounds P the same way, line 153-155);
+//  * the softmax runs beside the MFMAs: the 64 keys are two blocks of 32,
+//    block 0's exponentials issue between block 1's score MFMAs and block
+//    1's between block 0's P.V MFMAs.  They use the running max as it is,
+//    without a look at the new scores: a row's maximum would have to wait
+//    for all of the tile's scores before the first exponential.  The row
+//    sum that the block needs anyway tells afterwards whether that was good
+//    enough (every P is at most the sum): above kMaxBlockSum, or infinite,
+//    the block's maximum is taken and its exponentials are redone before
+//    P.V reads them.  Inputs with a tile-by-tile rising maximum take that
+//    path once per growth of the sum past 2^8.  Against a maximum per tile
+//    before the first exponential: 2048 x 8192 dense 252 -> 240 us, the last
+//    2048 tokens of a 32k prompt 963 -> 955 us, 8 x 512 73.3 -> 72.6 us, 4
+//    uneven sequences 51.9 -> 51.0 us (MFMA busy 56 -> 63 % dense, 59 -> 60 %
+//    long context); with zero inputs, where the clock does not fall under
+//    the MFMA load, the dense call gains 12 %;
 //  * causal tile skipping: a wave skips tiles past its largest visible key
-//    and applies the mask only on tiles that cross its smallest limit; the
-//    running max moves lazily (only when a row max grows by > 2^8), so O is
-//    rarely rescaled;
+//    and applies the mask only on tiles that cross its smallest limit;
 //  * tiles of one sequence are issued heaviest (last) first, and the work
 //    list is laid out so each XCD (workgroup id mod 8) gets a contiguous
 //    range of KV heads, keeping a head's pages in one L2;
@@ -61,6 +74,7 @@ constexpr int kStages = 2;
 constexpr int kRowBytes = kDimHead * 2;                // 256
 constexpr int kTileBytes = kKvTile * kRowBytes;        // 16 KB per K or V tile
 constexpr float kEmptyMaxP = -1.0e30f;
+constexpr float kMaxBlockSum = 256.0f;  // largest sum of a row's 16 exponentials in a lane before the running max moves
 constexpr int kSplitTries = 4;  // key-split granularities tried (T grows by half each time)
 
 // One page of zeros: the source of every copy whose block id lies outside
@@ -654,111 +668,120 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         constexpr bool kMayCopy = !std::is_same<decltype(copies_c), std::false_type>::value;
         const uint8_t* ks = smem[STAGE][0];
         const uint8_t* vs = smem[STAGE][1];
+        const int kr = lim - kb - 4 * h2;  // this row's limit relative to this lane's first key
 
-        // S^T blocks: keys kb + 32*kb2 + (0..31), queries = lanes (raw scores).
-        // The two blocks' MFMA chains alternate, and the K fragments of step
-        // kk are read at step kk - 2, so an MFMA does not wait out a full LDS
-        // read latency (with one chain after the other and one fragment
-        // register, every MFMA of the first chain did).
-        f32x16 sacc[2] = {f32x16{}, f32x16{}};
-        auto kfrag = [&](int kk, int kb2) {
-            const int chunk = (2 * kk + h2) ^ k_sw;
-            return *reinterpret_cast<const u32x4*>(ks + k_rd + kb2 * 32 * kRowBytes + (chunk << 4));
+        auto kfrag = [&](int n) __attribute__((always_inline)) {  // fragment of score MFMA n = 8 * block + kk
+            const int chunk = (2 * (n & 7) + h2) ^ k_sw;
+            return *reinterpret_cast<const u32x4*>(ks + k_rd + (n >> 3) * 32 * kRowBytes + (chunk << 4));
         };
-        u32x4 kf[3][2];
+        auto vfrag = [&](int n) __attribute__((always_inline)) {  // fragment of P.V MFMA n = 4 * ks2 + dt
+            u32x2 part[2];
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            kf[kk][0] = kfrag(kk, 0);
-            kf[kk][1] = kfrag(kk, 1);
-        }
-#pragma unroll
-        for (int kk = 0; kk < 8; ++kk) {
-            if (kk + 2 < 8) {
-                kf[(kk + 2) % 3][0] = kfrag(kk + 2, 0);
-                kf[(kk + 2) % 3][1] = kfrag(kk + 2, 1);
+            for (int half = 0; half < 2; ++half) {
+                const int key = 16 * (n >> 2) + 8 * half + v_key;
+                const int dim = 32 * (n & 3) + v_dim;
+                const int off = key * kRowBytes + ((((dim >> 3) ^ swz_v(key)) << 4) | ((dim & 4) << 1));
+                const v4i16 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(vs + off));
+                part[half] = __builtin_bit_cast(u32x2, r);
             }
-            sacc[0] = mfma32x32x16(E{}, kf[kk % 3][0], qreg[kk], sacc[0]);
-            sacc[1] = mfma32x32x16(E{}, kf[kk % 3][1], qreg[kk], sacc[1]);
+            return u32x4{part[0][0], part[0][1], part[1][0], part[1][1]};
+        };
+        // Values 2i and 2i + 1 of score block kb2 become two exponentials, one
+        // packed word of P and a term of the block's row sum.
+        float neg_m = -m_run;
+        auto soft = [&](const f32x16& sv, int i, u32x4 (&pw)[2], float& sum) __attribute__((always_inline)) {
+            float e[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                e[j] = fast_exp2(fmaf(sv[2 * i + j], scale, neg_m));
+            }
+            const uint32_t w = pack2(E{}, e[0], e[1]);
+            pw[i >> 2][i & 3] = w;
+            sum = sum2(E{}, w, sum);
+        };
+        // Before P.V reads a block's P: the mask, on tiles that cross a limit,
+        // and where some row's block sum passed kMaxBlockSum (out of line: it
+        // is rare) the running max moves to the block's and the exponentials
+        // are redone.
+        auto settle = [&](f32x16& sv, int kb2, u32x4 (&pw)[2], float& sum) __attribute__((always_inline)) {
+            if (kb + kKvTile > kfull_w) {  // wave-uniform: the tile crosses some row's limit
+#pragma unroll
+                for (int x = 0; x < 16; ++x) {
+                    const int rel = 32 * kb2 + 8 * (x >> 2) + (x & 3);
+                    sv[x] = rel < kr ? sv[x] : -INFINITY;
+                }
+                sum = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) soft(sv, i, pw, sum);
+            }
+            if (__builtin_expect(__ballot(sum > kMaxBlockSum) != 0, 0)) {
+                float mx = sv[0];
+#pragma unroll
+                for (int x = 1; x < 16; ++x) mx = fmaxf(mx, sv[x]);
+                float m_lo, m_hi;  // the row's two lane halves (keys 4*h2 + ...)
+                pair32(mx, m_lo, m_hi);
+                const float m_new = fmaxf(m_run, fmaxf(m_lo, m_hi) * scale);
+                const float alpha = fast_exp2(m_run - m_new);
+                m_run = m_new;
+                neg_m = -m_new;
+                l_run *= alpha;
+#pragma unroll
+                for (int dt = 0; dt < 4; ++dt) oacc[dt] *= alpha;
+                sum = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) soft(sv, i, pw, sum);
+            }
+            l_run += sum;
+        };
+        constexpr int kAhead = 4;  // fragments read ahead of their MFMA (3: 1 % slower on long context)
+        f32x16 s0 = f32x16{}, s1 = f32x16{};
+        u32x4 p0[2], p1[2];
+        float sum0 = 0.0f, sum1 = 0.0f;
+        u32x4 kf[kAhead + 1], vf[kAhead + 1];
+        // Each MFMA is fenced into one bundle with the fragment read ahead of
+        // it and its share of the other block's softmax: the compiler's own
+        // order puts the exponentials after the MFMAs (4-6 % slower).
+#pragma unroll
+        for (int n = 0; n < kAhead; ++n) kf[n] = kfrag(n);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int n = 0; n < 8; ++n) {
+            kf[(n + kAhead) % (kAhead + 1)] = kfrag(n + kAhead);
+            s0 = mfma32x32x16(E{}, kf[n % (kAhead + 1)], qreg[n], s0);
             if constexpr (kMayCopy) {
-                if (copies_c) copy_one(kk);  // the next tile's copy kk
+                if (copies_c && (n & 1)) copy_one(n >> 1);
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        // Keep that order: 4 reads, then 6 x (2 reads, 2 MFMAs), then 4 MFMAs.
-        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
 #pragma unroll
-        for (int g = 0; g < 6; ++g) {
-            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-        }
-        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-        // Accumulator i of block kb2 holds key kb + 32*kb2 + 8*(i/4) + 4*h2 + i%4.
-        float mx = -INFINITY;
-        if (kb + kKvTile > kfull_w) {  // wave-uniform: tile crosses some row's limit
-            const int kr = lim - kb - 4 * h2;  // key index relative to this lane's base
-#pragma unroll
-            for (int kb2 = 0; kb2 < 2; ++kb2) {
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int rel = 32 * kb2 + 8 * (i >> 2) + (i & 3);
-                    const float s = rel < kr ? sacc[kb2][i] : -INFINITY;
-                    sacc[kb2][i] = s;
-                    mx = fmaxf(mx, s);
-                }
+        for (int n = 8; n < 16; ++n) {
+            if (n + kAhead < 16) kf[(n + kAhead) % (kAhead + 1)] = kfrag(n + kAhead);
+            else vf[n + kAhead - 16] = vfrag(n + kAhead - 16);
+            s1 = mfma32x32x16(E{}, kf[n % (kAhead + 1)], qreg[n - 8], s1);
+            if constexpr (kMayCopy) {
+                if (copies_c && (n & 1)) copy_one(n >> 1);
             }
-        } else {
-#pragma unroll
-            for (int kb2 = 0; kb2 < 2; ++kb2) {
-#pragma unroll
-                for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sacc[kb2][i]);
-            }
+            if (n > 8) soft(s0, n - 9, p0, sum0);
+            if (n == 15) soft(s0, 7, p0, sum0);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        {
-            float m_lo, m_hi;  // the row's two lane halves (keys 4*h2 + ...)
-            pair32(mx, m_lo, m_hi);
-            mx = fmaxf(m_lo, m_hi) * scale;
+        // (keeps the exponentials above from being sunk below settle's branches)
+        asm volatile("" : "+v"(p0[0]), "+v"(p0[1]), "+v"(sum0));
+        settle(s0, 0, p0, sum0);
+#pragma unroll
+        for (int n = 0; n < 8; ++n) {
+            vf[(n + kAhead) % (kAhead + 1)] = vfrag(n + kAhead);
+            oacc[n & 3] = mfma32x32x16(E{}, vf[n % (kAhead + 1)], p0[n >> 2], oacc[n & 3]);
+            if (n > 0) soft(s1, n - 1, p1, sum1);
+            if (n == 7) soft(s1, 7, p1, sum1);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        // Lazy rescale: the running max m_run only moves when some row's
-        // max exceeds it by more than 8 (log2 units), so exponentials stay
-        // <= 2^8 and O is rarely rescaled.
-        if (__ballot(mx > m_run + 8.0f)) {
-            const float m_new = fmaxf(m_run, mx);
-            const float alpha = fast_exp2(m_run - m_new);
-            m_run = m_new;
-            l_run *= alpha;
+        asm volatile("" : "+v"(p1[0]), "+v"(p1[1]), "+v"(sum1));
+        settle(s1, 1, p1, sum1);
 #pragma unroll
-            for (int dt = 0; dt < 4; ++dt) oacc[dt] *= alpha;
-        }
-        const float neg_m = -m_run;
-
-        // P^T as the B operand: k-slot j of lane half h2 in step ks is key
-        // kb + 16*ks + 8*(j/4) + 4*h2 + j%4.  The row sum adds the rounded
-        // P values the MFMA consumes.
-        u32x4 pb[4];
-#pragma unroll
-        for (int ks2 = 0; ks2 < 4; ++ks2) {
-            float pf[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) pf[j] = fast_exp2(fmaf(sacc[ks2 >> 1][8 * (ks2 & 1) + j], scale, neg_m));
-            pb[ks2] = pack8(E{}, pf);
-            l_run = sum8(E{}, pb[ks2], l_run);
-        }
-
-#pragma unroll
-        for (int ks2 = 0; ks2 < 4; ++ks2) {
-#pragma unroll
-            for (int dt = 0; dt < 4; ++dt) {
-                u32x2 part[2];
-#pragma unroll
-                for (int half = 0; half < 2; ++half) {
-                    const int key = 16 * ks2 + 8 * half + v_key;
-                    const int dim = 32 * dt + v_dim;
-                    const int off = key * kRowBytes + ((((dim >> 3) ^ swz_v(key)) << 4) | ((dim & 4) << 1));
-                    const v4i16 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(vs + off));
-                    part[half] = __builtin_bit_cast(u32x2, r);
-                }
-                const u32x4 va = u32x4{part[0][0], part[0][1], part[1][0], part[1][1]};
-                oacc[dt] = mfma32x32x16(E{}, va, pb[ks2], oacc[dt]);
-            }
+        for (int n = 8; n < 16; ++n) {
+            if (n + kAhead < 16) vf[(n + kAhead) % (kAhead + 1)] = vfrag(n + kAhead);
+            oacc[n & 3] = mfma32x32x16(E{}, vf[n % (kAhead + 1)], p1[(n >> 2) - 2], oacc[n & 3]);
         }
     };
 

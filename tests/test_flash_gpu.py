@@ -117,3 +117,24 @@ def test_dense_errors(C, gpu):
         C.FlashAttentionWarpCuda(q.float(), q.float(), q.float())
     with pytest.raises(RuntimeError):
         C.FlashAttentionWarpCuda(q[..., :64].contiguous(), q[..., :64].contiguous(), q[..., :64].contiguous())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("jump", [3.0, 7.0, 40.0, 200.0])
+@pytest.mark.parametrize("at", [0, 31, 32, 63, 64, 95, 96, 150])
+def test_dense_attention_rising_scores(C, gpu, dtype, jump, at):
+    """Scores of some rows jump at key ``at`` (first and last key of both 32-key blocks of a tile): below,
+    just above and far above the kernel's limit on a block's sum, and past what exp2 holds (the jump is in
+    log2 units, times 1, -1 or 0 by row), on top of random scores.  Bounds as everywhere (the inputs are
+    rounded to the storage type before the oracle sees them)."""
+    q = rand((1, 4, 70, 128), dtype, 1)
+    k = rand((1, 2, 200, 128), dtype, 2)
+    v = rand((1, 2, 200, 128), dtype, 3)
+    q[:, :, 0::3, 0] = 16.0
+    q[:, :, 1::3, 0] = -16.0
+    q[:, :, 2::3, 0] = 0.0
+    k[..., 0] = 0.0
+    k[:, :, at:, 0] = jump * np.log(2.0) * np.sqrt(128.0) / 16.0
+    out = C.FlashAttentionWarpCuda(q.to(gpu), k.to(gpu), v.to(gpu))
+    torch.cuda.synchronize()
+    assert_close(out, oa.dense_attention(np64(q), np64(k), np64(v)), dtype, f"jump {jump} at key {at}")
