@@ -131,9 +131,9 @@ int femto_paged_attention_gemv_noalloc(
  * takes it; it only bounds how many sequences may have exactly one token.
  * workspace may be NULL.  With a workspace of at least
  * femto_paged_attention_gemm_workspace_size() bytes (256-byte aligned; its
- * first femto_paged_attention_gemm_split_bytes() bytes, the key-split
- * counters, zero-filled before the first use, and every call leaves them
- * zero-filled):
+ * first femto_paged_attention_gemm_split_bytes() bytes, the counters of the
+ * key split and of the decode rows' merge, zero-filled before the first use,
+ * and every call leaves them zero-filled):
  *  - the query tiles of sequences much longer than the average are split
  *    over their keys and merged within the launch, so a few long sequences
  *    do not set the length of the call;
@@ -142,8 +142,9 @@ int femto_paged_attention_gemv_noalloc(
  *    kernel's wave workers (the rest of the workspace holds their partial
  *    states) and the MFMA tiles skip them; the workers share the tiles'
  *    launch (a separate decode launch first when n_heads / n_kv_heads is a
- *    multiple of 8) and a small merge launch follows.  Without a workspace
- *    the MFMA kernel computes every row.
+ *    multiple of 8).  Where the possible rows are few they merge their
+ *    partials in that launch, else a small merge launch follows.  Without a
+ *    workspace the MFMA kernel computes every row.
  * Every launch goes on `stream`.  Calls that may overlap (other streams)
  * must not share a workspace. */
 int femto_paged_attention_gemm(
@@ -160,7 +161,7 @@ int femto_paged_attention_gemm(
     void* stream);
 
 /* Bytes of the optional workspace of femto_paged_attention_gemm: the
- * key-split part (one counter and one 66 KiB partial slot per workgroup the
+ * key-split part (two counters and one 66 KiB partial slot per workgroup the
  * current device holds at once, 2 per CU, independent of the batch) plus,
  * when the sizes allow one-token sequences, the decode rows' partial states
  * (num_seqs x n_heads x slots of 130 floats, slots set by the table width
@@ -170,8 +171,8 @@ size_t femto_paged_attention_gemm_workspace_size(int num_seqs, int num_tokens, i
                                                  int n_kv_heads, int num_pages_per_seq);
 
 /* Leading bytes of that workspace that must be zero-filled before its first
- * use: the key-split counters (the partial slots behind them and the
- * decode-row part need no initialisation).  No counterpart in the
+ * use: the counters (the partial slots behind them and the decode-row part
+ * need no initialisation).  No counterpart in the
  * reference. */
 size_t femto_paged_attention_gemm_split_bytes(void);
 

@@ -240,6 +240,34 @@ __device__ __forceinline__ int decode_len(const DecodeArgs& a, int b) {
     return len;
 }
 
+// Merge the four DPP rows' softmax states (same dims, different keys): rows
+// 0+1 and 2+3, then the two halves; every lane of a pair ends with the pair's
+// state (the first row's terms first, as row 0 computes them).
+template <int NREP>
+__device__ __forceinline__ void merge_dpp_rows(float (&m)[NREP], float (&l)[NREP], float (&acc)[NREP][8]) {
+    auto merge_pair = [&](auto pair) {
+#pragma unroll
+        for (int r = 0; r < NREP; ++r) {
+            float m0, m1, l0, l1;
+            pair(m[r], m0, m1);
+            pair(l[r], l0, l1);
+            const float mn = fmaxf(m0, m1);
+            const float f0 = fast_exp2(m0 - mn);
+            const float f1 = fast_exp2(m1 - mn);
+            l[r] = l0 * f0 + l1 * f1;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                float a0, a1;
+                pair(acc[r][e], a0, a1);
+                acc[r][e] = a0 * f0 + a1 * f1;
+            }
+            m[r] = mn;
+        }
+    };
+    merge_pair([](float x, float& a, float& b) { pair16(x, a, b); });
+    merge_pair([](float x, float& a, float& b) { pair32(x, a, b); });
+}
+
 // Softmax state of query heads h0 .. h0+NREP-1 of sequence b over pages
 // [lp0, lp0 + n) of its kv_len keys (query row qrow): the running max m
 // (log2 units), the row sum l and the 8 unnormalised accumulators of this
@@ -397,30 +425,111 @@ __device__ __forceinline__ void decode_segment(const DecodeArgs& a, int b, int k
         }
     }
 
-    // Merge the four DPP rows (same dims, different keys): rows 0+1 and
-    // 2+3, then the two halves; every lane of a pair ends with the pair's
-    // state (the first row's terms first, as row 0 computes them).
-    auto merge_pair = [&](auto pair) {
+    merge_dpp_rows<NREP>(m, l, acc);
+}
+
+// Normalised rows of query heads h0 .. h0+NREP-1 (every lane holds the state
+// for its dims); head r is written by DPP row r mod 4.
+template <typename E, int NREP, bool FULL>
+__device__ __forceinline__ void store_rows(const DecodeArgs& a, int row, int h0, const float (&l)[NREP],
+                                           const float (&acc)[NREP][8]) {
+    const int lane = threadIdx.x & 63, rg = lane >> 4, c = lane & 15;
+    char* out = reinterpret_cast<char*>(a.out);
+#pragma unroll
+    for (int r = 0; r < NREP; ++r) {
+        if (rg != (r & 3)) continue;
+        const int64_t o = (int64_t)(h0 + r) * a.out_stride_head + (int64_t)row * a.out_stride_seq;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int d = RowSlice<E>::dim(c, e);
+            if (FULL || d < a.head_dim) store_elem<E>(out, o + d, acc[r][e] / l[r]);
+        }
+    }
+}
+
+// A cut sequence's segment in a launch that merges by itself
+// (a.merge_counters): its partial goes out with system-scope stores (written
+// through to memory), then the wave counts itself in; the last of the
+// sequence's `count` waves reads all partials with system-scope loads, merges
+// them (slots dealt over the four DPP rows) and writes the output rows.  The
+// counter is back to zero afterwards.
+template <typename E, int NREP, bool FULL>
+__device__ __forceinline__ void publish_and_merge(const DecodeArgs& a, int b, int grp, int row, int h0, int slot_in,
+                                                  int count_in, const float (&m)[NREP], const float (&l)[NREP],
+                                                  const float (&acc)[NREP][8]) {
+    typedef unsigned u32x4v __attribute__((ext_vector_type(4)));
+    const int lane = threadIdx.x & 63, rg = lane >> 4, c = lane & 15;
+    const int slot = __builtin_amdgcn_readfirstlane(slot_in), count = __builtin_amdgcn_readfirstlane(count_in);
+    // One descriptor for each array; the offsets stay inside it (the launcher
+    // keeps num_seqs * n_heads * max_slots small enough for 32-bit bytes).
+    const auto ra = __builtin_amdgcn_make_buffer_rsrc(a.part_acc, (short)0, 0x7fffffff, 0x00020000);
+    const auto rm = __builtin_amdgcn_make_buffer_rsrc(a.part_ml, (short)0, 0x7fffffff, 0x00020000);
+    auto slot_of = [&](int r, int i) { return (b * a.n_heads + h0 + r) * a.max_slots + i; };
+    if (rg == 0) {
 #pragma unroll
         for (int r = 0; r < NREP; ++r) {
-            float m0, m1, l0, l1;
-            pair(m[r], m0, m1);
-            pair(l[r], l0, l1);
-            const float mn = fmaxf(m0, m1);
-            const float f0 = fast_exp2(m0 - mn);
-            const float f1 = fast_exp2(m1 - mn);
-            l[r] = l0 * f0 + l1 * f1;
+            const int sl = slot_of(r, slot);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                float a0, a1;
-                pair(acc[r][e], a0, a1);
-                acc[r][e] = a0 * f0 + a1 * f1;
-            }
-            m[r] = mn;
+            for (int h = 0; h < 2; ++h)
+                __builtin_amdgcn_raw_buffer_store_b128(
+                    u32x4v{__float_as_uint(acc[r][4 * h]), __float_as_uint(acc[r][4 * h + 1]),
+                           __float_as_uint(acc[r][4 * h + 2]), __float_as_uint(acc[r][4 * h + 3])},
+                    ra, (sl * kDimHead + RowSlice<E>::dim(c, 4 * h)) * 4, 0, 0x11);
+            if (c == 0)
+                __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(m[r]), __float_as_uint(l[r])}, rm, sl * 8, 0,
+                                                      0x11);
         }
-    };
-    merge_pair([](float x, float& a, float& b) { pair16(x, a, b); });
-    merge_pair([](float x, float& a, float& b) { pair32(x, a, b); });
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the partial is in memory before the count goes up
+    int* counter = a.merge_counters + b * a.grid_heads + grp;
+    int old = 0;
+    if (lane == 0) old = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__builtin_amdgcn_readfirstlane(old) != count - 1) return;  // another wave merges
+    if (lane == 0) __hip_atomic_exchange(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("" ::: "memory");
+    float M[NREP], L[NREP], A[NREP][8];
+#pragma unroll
+    for (int r = 0; r < NREP; ++r) {
+        M[r] = kEmptyMax;
+        L[r] = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) A[r][e] = 0.0f;
+    }
+    constexpr int kU = 4;  // slots per DPP row and round, their loads in flight together
+#pragma unroll 1
+    for (int i0 = 0; i0 < count; i0 += 4 * kU) {
+        u32x2 ml[kU][NREP];
+        u32x4v v[kU][NREP][2];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const int i = min(i0 + 4 * u + rg, count - 1);  // past the end: the last slot again, with weight 0
+#pragma unroll
+            for (int r = 0; r < NREP; ++r) {
+                const int sl = slot_of(r, i);
+                ml[u][r] = __builtin_amdgcn_raw_buffer_load_b64(rm, sl * 8, 0, 0x11);
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    v[u][r][h] = __builtin_amdgcn_raw_buffer_load_b128(
+                        ra, (sl * kDimHead + RowSlice<E>::dim(c, 4 * h)) * 4, 0, 0x11);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const bool live = i0 + 4 * u + rg < count;
+#pragma unroll
+            for (int r = 0; r < NREP; ++r) {
+                const float ms = __uint_as_float(ml[u][r][0]);
+                const float mn = live ? fmaxf(M[r], ms) : M[r];
+                const float f0 = fast_exp2(M[r] - mn), f1 = live ? fast_exp2(ms - mn) : 0.0f;
+                L[r] = L[r] * f0 + __uint_as_float(ml[u][r][1]) * f1;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) A[r][e] = A[r][e] * f0 + __uint_as_float(v[u][r][e >> 2][e & 3]) * f1;
+                M[r] = mn;
+            }
+        }
+    }
+    merge_dpp_rows<NREP>(M, L, A);
+    store_rows<E, NREP, FULL>(a, row, h0, L, A);
 }
 
 // Load-balanced split-KV decode.  Every wave is an independent worker: the
@@ -432,7 +541,8 @@ __device__ __forceinline__ void decode_segment(const DecodeArgs& a, int b, int k
 // The waves of workgroup `block` (4 per workgroup, no barriers: a wave may
 // return on its own); used by the decode kernel and by the fused prefill
 // launch, whose first workgroups are decode workers.
-template <typename E, int NREP, bool FULL = true>
+// MAY_MERGE: built with the in-launch merge (used when a.merge_counters is set).
+template <typename E, int NREP, bool FULL, bool MAY_MERGE>
 __device__ __forceinline__ void decode_waves(const DecodeArgs& a, int block) {
     const int lane = threadIdx.x & 63;
     const int gw = block * 4 + (threadIdx.x >> 6);
@@ -445,6 +555,20 @@ __device__ __forceinline__ void decode_waves(const DecodeArgs& a, int block) {
     const int rg = lane >> 4;
     const int c = lane & 15;
     const int B = a.num_seqs;
+
+    if (MAY_MERGE && a.merge_counters && wi == 0) {
+        // Rows with no visible key, which no wave below meets: 0 / 0, as the
+        // merge launch writes them.
+        for (int i = lane; i < B; i += kWave) {
+            int row, len;
+            if (!decode_row_of(a, i, row, len) || len > 0) continue;
+            for (int r = 0; r < NREP; ++r)
+                for (int d = 0; d < a.head_dim; ++d)
+                    store_elem<E>(reinterpret_cast<char*>(a.out),
+                                  (int64_t)(h0 + r) * a.out_stride_head + (int64_t)row * a.out_stride_seq + d,
+                                  __builtin_nanf(""));
+        }
+    }
 
     // Pass 1: total pages P and the longest sequence; slice length C.
     int total = 0, longest = 0;
@@ -513,6 +637,14 @@ __device__ __forceinline__ void decode_waves(const DecodeArgs& a, int block) {
 
         // Partial state of this segment.
         const int slot = wi - S / C;
+        if (MAY_MERGE && a.merge_counters) {
+            const int count = (S + npg - 1) / C - S / C + 1;  // waves that hold a part of the sequence
+            if (count == 1) store_rows<E, NREP, FULL>(a, qrow, h0, l, acc);
+            else publish_and_merge<E, NREP, FULL>(a, b, grp, qrow, h0, slot, count, m, l, acc);
+            x = S + lp1;
+            ++b;
+            continue;
+        }
         if (rg == 0) {
 #pragma unroll
             for (int r = 0; r < NREP; ++r) {

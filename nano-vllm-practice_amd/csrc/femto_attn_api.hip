@@ -455,6 +455,21 @@ int femto_paged_attention_gemm(int dtype, const void* q, int64_t q_stride_head, 
             // launch as the tiles, which fill the CU slots beside them; else
             // the decode kernel runs first.
             const femto::DecodePlan plan = gemm_decode_plan(n_heads, n_kv_heads, num_pages_per_seq);
+            decode_rows = femto::decode_rows_bound(num_seqs, num_tokens, max_q_len);
+            // Few possible one-token sequences (often none: chunks of uneven
+            // lengths leave the bound above zero): the workers merge their
+            // partials in the launch, the last wave of each (sequence, KV
+            // head group) folding the others', so no merge launch follows.
+            // That serial tail beats the launch while the merges are at most
+            // a quarter of the ~1024 worker waves: 1024 new tokens beside
+            // 1 / 16 / 31 rows on 8 KV heads 40.5 -> 38.5, 65.3 -> 57.8,
+            // 72.9 -> 68.8 us; 4 uneven chunks without rows 51.5 -> 50.1 us;
+            // 48 rows 93.6 -> 94.0 and, beside 64 tokens, 44.5 -> 45.2 us.
+            // Groups of four heads keep the merge launch: the fold costs the
+            // tiles' kernel its registers (256, and 2x slower workers).
+            const int group = femto::prefill_group(a.n_rep);
+            const int64_t groups = n_heads / group;
+            const bool few = group <= 2 && decode_rows * groups <= resident / 2 && num_seqs * groups <= resident;
             femto::DecodeArgs d = femto::decode_args(
                 plan, q, q_stride_head, q_stride_token, out, out_stride_head, out_stride_token, k_pool, v_pool,
                 num_blocks, n_kv_heads, head_dim, pool_stride_block, pool_stride_head, pool_stride_row,
@@ -462,9 +477,9 @@ int femto_paged_attention_gemm(int dtype, const void* q, int64_t q_stride_head, 
                 static_cast<char*>(workspace) + split_bytes);
             d.cu_seqlens = cu_seqlens;
             d.positions = positions;
+            if (few) d.merge_counters = a.counters + resident;
             a.skip_decode_rows = 1;
-            decode_rows = femto::decode_rows_bound(num_seqs, num_tokens, max_q_len);
-            if (plan.nrep_tile == femto::prefill_group(a.n_rep)) {
+            if (plan.nrep_tile == group) {
                 a.decode_blocks = femto::decode_worker_blocks(d);
                 if (a.decode_blocks <= 0) return fail(FEMTO_ERR_HIP, "paged_attention_gemm: device query");
                 a.dec = d;

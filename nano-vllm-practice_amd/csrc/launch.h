@@ -39,6 +39,10 @@ struct DecodeArgs {
     // j < min(kv_lens[b], positions[row] + 1).
     const int32_t* cu_seqlens;
     const int32_t* positions;
+    // Decode rows only: one zeroed counter per (sequence, KV head group); the
+    // waves of a cut sequence merge their partials themselves and no merge
+    // launch follows.  Null: partials only.
+    int* merge_counters;
 };
 
 // Compute units of the current device, queried once per device (safe to call
@@ -106,6 +110,8 @@ struct PrefillArgs {
 constexpr int kMaxPieces = 8;
 constexpr int kPartSlotBytes = 4 * 64 * 64 * 4 + 4 * 64 * 8;
 hipError_t prefill_resident_workgroups(int& resident);
+// Counters at the front of the workspace: one per resident workgroup for the
+// key split, then as many for the decode rows' in-launch merge.
 size_t prefill_counter_bytes(int resident);
 size_t prefill_workspace_bytes(int resident);
 

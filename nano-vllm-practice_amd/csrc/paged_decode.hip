@@ -34,7 +34,7 @@ namespace femto {
 
 template <typename E, int NREP, bool FULL>
 __global__ __launch_bounds__(256) void paged_decode_kernel(DecodeArgs a) {
-    decode_waves<E, NREP, FULL>(a, blockIdx.x);
+    decode_waves<E, NREP, FULL, false>(a, blockIdx.x);
 }
 
 // One-launch decode for calls of short contexts: one workgroup of W waves per

@@ -274,7 +274,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         // the decode kernel would use for this head ratio); they are
         // dispatched first, one per CU, and the tiles fill the other slots.
         if (lin < a.decode_blocks) {
-            decode_waves<E, G, FULLD>(a.dec, lin);
+            decode_waves<E, G, FULLD, (G <= 2)>(a.dec, lin);
             return;
         }
         lin -= a.decode_blocks;  // a multiple of 8: the XCD of a tile is unchanged
@@ -1072,8 +1072,10 @@ hipError_t prefill_resident_workgroups(int& resident) {
 }
 
 // A split call has at most `resident` pieces in all: one counter and one
-// partial slot per resident workgroup, whatever the batch.
-size_t prefill_counter_bytes(int resident) { return ((size_t)resident * sizeof(int) + 255) & ~(size_t)255; }
+// partial slot per resident workgroup, whatever the batch.  (As many counters
+// again for the decode rows' merge: a call that needs more takes the merge
+// launch.)
+size_t prefill_counter_bytes(int resident) { return ((size_t)resident * 2 * sizeof(int) + 255) & ~(size_t)255; }
 
 size_t prefill_workspace_bytes(int resident) {
     return resident > 0 ? prefill_counter_bytes(resident) + (size_t)resident * kPartSlotBytes : 0;
@@ -1116,7 +1118,7 @@ hipError_t launch_paged_prefill(int dtype, PrefillArgs a, int num_tokens, int de
         }
     }
     hipError_t e = launch_dtype<true>(dtype, G, a, st);
-    if (e == hipSuccess && a.decode_blocks > 0) e = launch_paged_decode_merge(dtype, a.dec, a.num_seqs, st);
+    if (e == hipSuccess && a.decode_blocks > 0 && !a.dec.merge_counters) e = launch_paged_decode_merge(dtype, a.dec, a.num_seqs, st);
     return e;
 }
 

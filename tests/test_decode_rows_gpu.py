@@ -124,3 +124,46 @@ def test_all_decode_rows_call(ops, gpu, monkeypatch):
         _no_workspace(m)
         mfma = _gemm(ops, q, meta, wd, gpu)
     assert_close(mfma, want, torch.bfloat16, "all decode rows, MFMA kernel")
+
+
+@pytest.mark.parametrize("heads", [(16, 8), (16, 16), (2, 1), (3, 3)], ids=str)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("dim", [128, 48])
+def test_rows_merged_in_the_launch(ops, gpu, heads, dtype, dim):
+    """One or two query heads per KV head and few rows: the workers of a cut row merge its partials in the
+    launch (rows inside one slice, cut in two and in many, cut contexts and rows that see nothing), three
+    times over from the counters that the last call left, then by graph replays."""
+    from femtovllm import _C
+
+    chunks = [(0, 1), (15, 1), (16, 1), (3000, 1), (100, 33), (63, 1), (20, 0), (700, 1), (511, 1), (0, 2)]
+    w = workloads.make_paged_workload("merge_in_launch", chunks, *heads, seed=41, dtype=dtype, head_dim=dim)
+    q, meta = w.gemm_call(device=gpu)
+    wd = w.to(gpu)
+    pos, kv, cu = list(meta.raw_positions), meta.kv_lens.tolist(), meta.raw_cu_seqlens
+    pos[cu[5]] = -1  # sees nothing
+    pos[cu[7]] = 333  # cut inside the context
+    kv[8] = 0  # empty context
+    positions = torch.tensor(pos, dtype=torch.int32, device=gpu)
+    kv_lens = torch.tensor(kv, dtype=torch.int32, device=gpu)
+    want = _oracle(q, meta, w, kv, pos)
+    what = f"rows merged in the launch {heads} {dtype} {dim}"
+    call = lambda: _gemm(ops, q, meta, wd, gpu, kv_lens=kv_lens, positions=positions)
+    for _ in range(3):
+        assert_close(call(), want, dtype, what)
+    zeros = int(_C._lib.femto_paged_attention_gemm_split_bytes())
+    for (dev, _), ws in _C._prefill_workspaces.items():
+        off = -ws.data_ptr() % 256
+        assert dev != gpu.index or int(torch.count_nonzero(ws[off:off + zeros])) == 0
+    qd, side, graph = q.to(gpu), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    args = (qd, wd.k_pool, wd.v_pool, meta.cu_seqlens, meta.max_q_len, meta.Q_TILE_SIZE, meta.cu_q_tiles,
+            meta.q_tile_to_seq_idx, meta.block_tables, kv_lens, positions)
+    with torch.cuda.stream(side):
+        ops.paged_attention_gemm(*args)  # this stream's workspace
+        side.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            out = ops.paged_attention_gemm(*args)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_close(out, want, dtype, what + ", graph")
