@@ -1,10 +1,11 @@
-"""Build libfemto_attn.so for gfx950 with hipcc (in-tree).
+"""Build libfemto_attn.so for gfx950 with hipcc, and femto_native.so with g++ (in-tree).
 
     python nano-vllm-practice_amd/build.py            # build
     python nano-vllm-practice_amd/build.py --verbose  # print the hipcc line
 
-The library lands in ``femtovllm/_lib/libfemto_attn.so`` next to the Python
-package that loads it.  Code objects are pinned to code-object version 5 so
+The libraries land in ``femtovllm/_lib/`` next to the Python package that
+loads them.  libfemto_attn.so holds the kernels and the C ABI; femto_native.so
+(host code only, against torch's headers) makes the Python layer's calls.  Code objects are pinned to code-object version 5 so
 the HIP runtime bundled with PyTorch-ROCm 7.0 loads them, and packed-fp32
 instruction selection is disabled for the device pass.
 """
@@ -22,6 +23,7 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(ROOT, "include")
 OUT_DIR = os.path.join(HERE, "femtovllm", "_lib")
 LIB = os.path.join(OUT_DIR, "libfemto_attn.so")
+NATIVE = os.path.join(OUT_DIR, "femto_native.so")
 
 SOURCES = ["femto_attn_api.hip", "paged_decode.hip", "paged_prefill.hip", "kv_cache_write.hip", "qk_norm_rope.hip", "varlen_metadata.hip"]
 
@@ -45,8 +47,25 @@ def hipcc() -> str:
     raise RuntimeError("hipcc not found (ROCm is required to build libfemto_attn.so)")
 
 
+def native_command(out: str) -> list:
+    import sysconfig
+
+    from torch.utils import cpp_extension
+
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(hipcc())))
+    include = [INCLUDE, *cpp_extension.include_paths(), sysconfig.get_paths()["include"], os.path.join(rocm, "include")]
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
+            *[f"-I{d}" for d in include], os.path.join(CSRC, "native_calls.cpp"), "-o", out,
+            *[f"-L{d}" for d in cpp_extension.library_paths()], "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+
+
 def build(verbose: bool = False) -> str:
     os.makedirs(OUT_DIR, exist_ok=True)
+    native_tmp = NATIVE + ".tmp"
+    native_cmd = native_command(native_tmp)
+    if verbose:
+        print(" ".join(native_cmd), flush=True)
+    native = subprocess.Popen(native_cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     tmp = LIB + ".tmp"
     cmd = [hipcc(), *HIPCC_FLAGS, "-I", INCLUDE, "-I", CSRC,
            *[os.path.join(CSRC, s) for s in SOURCES], "-o", tmp]
@@ -61,7 +80,11 @@ def build(verbose: bool = False) -> str:
         raise RuntimeError(f"hipcc failed ({res.returncode}):\n{errs}")
     if verbose and errs.strip():
         print(errs, flush=True)
+    native_out = native.communicate()[0]
+    if native.returncode != 0:
+        raise RuntimeError(f"g++ failed ({native.returncode}):\n{native_out}")
     os.replace(tmp, LIB)
+    os.replace(native_tmp, NATIVE)
     return LIB
 
 

@@ -29,11 +29,15 @@ exactly 128, as the reference's.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import torch
 
-_LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "libfemto_attn.so")
+_LIB_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib")
+_LIB_PATH = os.path.join(_LIB_DIR, "libfemto_attn.so")
+_NATIVE_PATH = os.path.join(_LIB_DIR, "femto_native.so")
 
 
 def _load() -> ctypes.CDLL:
@@ -88,6 +92,28 @@ def _load() -> ctypes.CDLL:
 
 
 _lib = _load()
+
+
+def _load_native():
+    """csrc/native_calls.cpp: the calls below with their checks and tensor handling in C++, over the
+    library that ``_lib`` loaded.  Each returns None where it does not take a call (nothing has been
+    launched then), and the Python code after it does, with its own checks, errors and allocations."""
+    if not os.path.exists(_NATIVE_PATH):
+        raise ImportError(
+            "femtovllm HIP backend is not built: missing "
+            f"{_NATIVE_PATH}\nBuild it with: python nano-vllm-practice_amd/build.py"
+        )
+    loader = importlib.machinery.ExtensionFileLoader("femto_native", _NATIVE_PATH)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("femto_native", loader))
+    loader.exec_module(module)
+    names = ("femto_attn_last_error", "femto_paged_attention_gemv", "femto_paged_attention_gemv_workspace_size",
+             "femto_paged_attention_gemm", "femto_paged_attention_gemm_workspace_size",
+             "femto_qk_norm_rope_cache_write", "femto_flash_attention")
+    module.bind({n: ctypes.cast(getattr(_lib, n), ctypes.c_void_p).value for n in names})
+    return module
+
+
+_native = _load_native()
 
 kMaxKVLenNonSplit = int(_lib.femto_attn_max_kv_len_non_split())
 kKVLenPerPage = int(_lib.femto_attn_kv_len_per_page())
@@ -157,6 +183,9 @@ def _prefill_workspace(device: torch.device, num_seqs: int, num_tokens: int, max
     return _cached_workspace(_prefill_workspaces, device, nbytes, zero=True)
 
 
+_stream_prefill_workspace = _prefill_workspace  # a caller that replaces _prefill_workspace gets the Python path
+
+
 def _check_paged(fn, q, k_pool, v_pool, tables, kv_lens, require_contiguous_q, decode=False):
     for name, t in (("q", q), ("k_pool", k_pool), ("v_pool", v_pool)):
         _check(t.is_cuda, f"{fn}: {name} must be a GPU tensor")
@@ -193,6 +222,10 @@ def _paged_attention_gemv(q, k_pool, v_pool, kv_page_tables, kv_lens, max_kv_len
     """Decode through the C ABI.  ``max_kv_len_limit`` is the reference's
     ``kMaxKVLenNonSplit`` check (paged_attention_gemv.cu:271-274); ``None``
     lifts it, since the kernel splits contexts of any length over waves."""
+    out = _native.gemv(q, k_pool, v_pool, kv_page_tables, kv_lens, max_kv_len, require_contiguous_q,
+                       max_kv_len_limit, _workspaces)
+    if out is not None:
+        return out
     fn = "PagedAttentionGemvCuda"
     _check_paged(fn, q, k_pool, v_pool, kv_page_tables, kv_lens, require_contiguous_q, decode=True)
     n_heads, num_seqs, dim = q.shape
@@ -223,6 +256,11 @@ def _paged_attention_gemv(q, k_pool, v_pool, kv_page_tables, kv_lens, max_kv_len
 
 def _paged_attention_gemm(q, k_pool, v_pool, cu_seqlens, max_q_len, kv_page_tables, kv_lens, positions,
                           require_contiguous_q=True):
+    if _prefill_workspace is _stream_prefill_workspace:
+        out = _native.gemm(q, k_pool, v_pool, cu_seqlens, max_q_len, kv_page_tables, kv_lens, positions,
+                           require_contiguous_q, _prefill_workspaces)
+        if out is not None:
+            return out
     fn = "PagedAttentionGemmCuda"
     _check_paged(fn, q, k_pool, v_pool, kv_page_tables, kv_lens, require_contiguous_q)
     for name, t in (("cu_seqlens", cu_seqlens), ("positions", positions)):
@@ -311,6 +349,10 @@ def _kv_cache_write(k, v, k_pool, v_pool, positions, kv_page_tables, cu_seqlens=
 def _qk_norm_rope_cache_write(q, k, v, q_weight, k_weight, eps, cos, sin, positions, k_pool, v_pool,
                               kv_page_tables, cu_seqlens=None, max_q_len=1, out=None):
     """RMSNorm + RoPE of q and k, q to ``out``, rotated k and v into the pools; returns ``out``."""
+    done = _native.prologue(q, k, v, q_weight, k_weight, eps, cos, sin, positions, k_pool, v_pool, kv_page_tables,
+                            cu_seqlens, max_q_len, out)
+    if done is not None:
+        return done
     fn = "qk_norm_rope_cache_write"
     for name, t in (("q", q), ("k", k), ("v", v), ("q_weight", q_weight), ("k_weight", k_weight),
                     ("cos", cos), ("sin", sin), ("k_pool", k_pool), ("v_pool", v_pool)):
@@ -406,6 +448,9 @@ def PagedAttentionGemmCuda(q, k_pool, v_pool, cu_seqlens, max_q_len, kv_page_tab
 
 def FlashAttentionWarpCuda(q, k, v):
     """Dense non-causal GQA attention, q (B, H, Tq, 128), k/v (B, KVH, Tkv, 128)."""
+    out = _native.flash(q, k, v)
+    if out is not None:
+        return out
     fn = "FlashAttentionWarpCuda"
     for name, t in (("q", q), ("k", k), ("v", v)):
         _check(t.is_cuda, f"{fn}: {name} must be a GPU tensor")
