@@ -41,10 +41,11 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(DecodeArgs a) {
 // (sequence, KV head group), wave w taking the w-th of W contiguous shares
 // of the sequence's pages; the waves fold their states through LDS and
 // write the normalised rows, so no workspace and no merge launch are needed.
-// Decode calls only (query row b, kv_lens[b] keys).  W = 4; calls with few
-// (sequence, query head) pairs run one query head per wave with W = 8, so
-// each wave walks half as many pages (a wave's page math, not the loads,
-// sets the length of such a call).
+// Decode calls only (query row b, kv_lens[b] keys).  W = 8 in calls of at most
+// one workgroup per CU, whose waves then walk half as many pages (the chain of
+// page loads and page math of a wave sets the length of such a call), else 4:
+// eight-wave workgroups would take more rounds (64 sequences of up to 512 keys
+// on 16/8 heads 18.6 us with four waves, 21.6 with eight).  decode_route picks.
 template <typename E, int NREP, bool FULL, int W>
 __global__ __launch_bounds__(64 * W) void paged_decode_single_kernel(DecodeArgs a) {
     __shared__ float s_ml[W][NREP][2];
@@ -199,15 +200,15 @@ hipError_t launch_paged_decode_merge(int dtype, const DecodeArgs& a, int num_seq
 template <typename E, int NREP, bool FULL>
 static hipError_t launch_t(DecodeArgs a, int num_seqs, bool single, hipStream_t st) {
     if (single) {
-        if constexpr (NREP == 1) {
+        const dim3 grid(num_seqs, a.grid_heads);
+        if constexpr (NREP == 1 || (NREP <= 4 && !std::is_same<E, F32>::value)) {
             if (a.single_waves == 8) {
-                hipLaunchKernelGGL((paged_decode_single_kernel<E, 1, FULL, 8>), dim3(num_seqs, a.grid_heads),
-                                   dim3(512), 0, st, a);
+                hipLaunchKernelGGL((paged_decode_single_kernel<E, NREP, FULL, 8>), grid, dim3(512), 0, st, a);
                 return hipGetLastError();
             }
         }
-        hipLaunchKernelGGL((paged_decode_single_kernel<E, NREP, FULL, 4>), dim3(num_seqs, a.grid_heads), dim3(256), 0,
-                           st, a);
+        if (a.single_waves != 4) return hipErrorInvalidValue;
+        hipLaunchKernelGGL((paged_decode_single_kernel<E, NREP, FULL, 4>), grid, dim3(256), 0, st, a);
         return hipGetLastError();
     }
     const int grid = decode_worker_blocks(a);

@@ -1,0 +1,59 @@
+"""The form a decode call takes by its shape (query heads per wave, waves, one launch or split).
+
+Batches at the edges of each choice (128 to 3072 workgroups, 256 to 1024 keys) against the oracle, and
+the calls that must stay on the one-launch kernel because they bring no workspace.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle.attention as oa
+from femtovllm import workloads
+from helpers import assert_close, np32, np64, np_tables
+
+pytestmark = pytest.mark.gpu
+
+# (heads, kv_heads, sequences): on both sides of the workgroup counts where the form changes
+SHAPES = [(16, 8, 16), (16, 8, 17), (16, 8, 32), (16, 8, 33), (32, 8, 32), (32, 8, 33), (64, 8, 8), (64, 8, 17),
+          (64, 8, 33), (64, 8, 65), (64, 8, 193), (16, 8, 8), (16, 8, 193), (4, 1, 65), (3, 3, 86), (24, 2, 11)]
+
+
+def _batch(heads, kv_heads, seqs, longest, dtype):
+    lens = [int(x) for x in np.random.default_rng(seqs).integers(1, 40, size=seqs)]
+    lens[seqs // 2] = longest
+    w = workloads.make_paged_workload("route", [(n - 1, 1) for n in lens], heads, kv_heads, seed=seqs, dtype=dtype)
+    return w
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("longest", [200, 300, 513, 900, 1025])
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_route_edges(ops, gpu, dtype, longest, shape):
+    w = _batch(*shape, longest, dtype)
+    q, meta = w.gemv_call(device=gpu)
+    wd = w.to(gpu)
+    out = ops.paged_attention_gemv(q.to(gpu), wd.k_pool, wd.v_pool, meta.block_tables, meta.kv_lens, meta.max_kv_len)
+    torch.cuda.synchronize()
+    want = oa.paged_decode(np64(q), np32(w.k_pool), np32(w.v_pool), np_tables(meta), meta.kv_lens.tolist())
+    assert_close(out, want, dtype, f"decode route {shape} {longest} {dtype}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_no_workspace_within_the_limit(gpu, dtype):
+    """A shape that would run split, called with no workspace: one launch, as before."""
+    from femtovllm import _C
+
+    w = _batch(64, 8, 193, 1000, dtype)
+    q, meta = w.gemv_call(device=gpu)
+    wd, q = w.to(gpu), q.to(gpu).contiguous()
+    out = torch.empty_like(q)
+    k, v, t = wd.k_pool, wd.v_pool, meta.block_tables
+    rc = _C._lib.femto_paged_attention_gemv(
+        _C._DTYPE[dtype], q.data_ptr(), q.stride(0), q.stride(1), out.data_ptr(), out.stride(0), out.stride(1), k.data_ptr(),
+        v.data_ptr(), *k.shape, *k.stride()[:3], t.data_ptr(), t.size(1), t.stride(0), meta.kv_lens.data_ptr(), q.size(1),
+        q.size(0), meta.max_kv_len, None, 0, _C._stream(q.device))
+    assert rc == 0, _C._lib.femto_attn_last_error().decode()
+    torch.cuda.synchronize()
+    want = oa.paged_decode(np64(q), np32(w.k_pool), np32(w.v_pool), np_tables(meta), meta.kv_lens.tolist())
+    assert_close(out, want, dtype, "no workspace")
