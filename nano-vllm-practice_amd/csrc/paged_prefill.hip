@@ -291,121 +291,51 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if constexpr (PAGED) {
         const int groups = a.n_kv_heads * a.head_groups;
         bool split = a.part != nullptr;
-        // Per-sequence sizes, loaded once: thread t keeps sequence t (the
-        // passes below reload only for sequences past the first 256).
-        int my_q0 = 0, my_ql = 0, my_kvl = 0, my_dec = 0;
-        if (tid < a.num_seqs) {
-            my_q0 = a.cu_seqlens[tid];
-            my_ql = a.cu_seqlens[tid + 1] - my_q0;
-            my_dec = a.skip_decode_rows && my_ql == 1;
-            if (my_dec) my_ql = 0;  // run by the decode kernel
-            my_kvl = a.kv_lens[tid];
-        }
-        auto seq_sizes = [&](int i, int& ql, int& kvl) {
-            if (i < 256) {
-                ql = my_ql;
-                kvl = my_kvl;
-            } else {
-                ql = a.cu_seqlens[i + 1] - a.cu_seqlens[i];
-                if (a.skip_decode_rows && ql == 1) ql = 0;
-                kvl = a.kv_lens[i];
-            }
+        auto pieces_of = [&](int kvl, int t) {
+            const int ub = kvl > 0 ? (kvl + kKvTile - 1) / kKvTile : 0;
+            return min(kMaxPieces, max(1, (2 * ub + t) / (2 * t)));
         };
-        // Pieces per query tile of sequence i: round(key tiles / T), at most
-        // kMaxPieces, where T0 is the estimated key tiles per resident
-        // workgroup of the whole call (query tile j of a chunk of ql tokens
-        // sees about kv_len - ql + BT (j+1) keys).  A sequence up to 1.5 times
-        // the average is not split.
-        int T0 = 0;
-        if (split) {
-            for (int base = 0; base < a.num_seqs; base += 256) {
-                const int i = base + tid;
-                int est = 0;
-                if (i < a.num_seqs) {
-                    int ql, kvl;
-                    seq_sizes(i, ql, kvl);
-                    if (ql > 0 && kvl > 0) {
-                        const int mean_keys = min(kvl, max(1, kvl - ql + (ql + BT) / 2));
-                        est = ((ql + BT - 1) / BT) * ((mean_keys + kKvTile - 1) / kKvTile);
-                    }
-                }
-                int tot[1] = {est};
-                block_reduce_n(tot, s_red);
-                T0 += tot[0];
+        // Key tiles of a sequence's query tiles, for the split estimate
+        // (query tile j of a chunk of ql tokens sees about kv_len - ql +
+        // BT (j+1) keys).
+        auto key_tiles = [&](int ql, int kvl) {
+            if (ql <= 0 || kvl <= 0) return 0;
+            const int mean_keys = min(kvl, max(1, kvl - ql + (ql + BT) / 2));
+            return ((ql + BT - 1) / BT) * ((mean_keys + kKvTile - 1) / kKvTile);
+        };
+        int w, seq_tile, ql_b;  // work item; its query tile (and piece) within the sequence; the sequence's tokens
+        if (a.num_seqs <= kWave) {
+            // Up to 64 sequences: lane i of every wave keeps sequence i, and
+            // each wave finds the work item by itself, with DPP sums and a
+            // ballot instead of three rounds through LDS and barriers (a
+            // 333-token prompt 14.3 -> 12.3 us, 12 chunks of 50-400 tokens 28.9 ->
+            // 27.1, 4 uneven 49.8 -> 47.8; the rules are those of the
+            // path below).
+            int q0 = 0, ql = 0, kvl = 0, dec = 0;
+            if (lane < a.num_seqs) {
+                q0 = a.cu_seqlens[lane];
+                ql = a.cu_seqlens[lane + 1] - q0;
+                kvl = a.kv_lens[lane];
+                dec = a.skip_decode_rows && ql == 1;
+                if (dec) ql = 0;  // run by the decode workers
             }
-            T0 = max(8, (int)(((int64_t)T0 * groups + a.resident - 1) / a.resident));
-        }
-        // Pieces only pay off in workgroup slots that would otherwise idle
-        // (a second round of pieces costs more than it balances): of the
-        // candidates T0, 1.5 T0, 2.25 T0, 3.375 T0 (fewer sequences split
-        // each time) the first whose pieces all fit in the resident slots at
-        // once is taken, else the call runs unsplit.
-        int w = 0;
-        if (tid == 0) s_seq = -1;
-        if (!split && a.num_seqs <= 256) {
-            // Unsplit call, one sequence per thread: a single scan gives both
-            // the work total and each sequence's first query tile.
-            const int nt = tid < a.num_seqs && my_ql > 0 ? (my_ql + BT - 1) / BT : 0;
-            // beside decode workers with one-token sequences the copies are spread
-            if constexpr (FUSED) spread = __syncthreads_or(my_dec) != 0;
-            int total;
-            const int incl = block_incl_scan(nt, s_red, total);
-            const int work = groups * total;
-            const int per_xcd = (work + 7) >> 3;
-            if ((lin >> 3) >= per_xcd) return;
-            w = (lin & 7) * per_xcd + serpentine(lin >> 3, per_xcd, a.resident >> 4);
-            if (w >= work) return;
-            grp = w / total;
-            tile_lin = w - grp * total;
-            if (nt > 0 && tile_lin >= incl - nt && tile_lin < incl) {
-                s_seq = tid;
-                s_ltile = tile_lin - (incl - nt);
-                s_kend[0] = my_q0;  // q_begin (s_kend is rewritten below)
-                s_kend[1] = my_ql;
-                s_kend[2] = my_kvl;
-                s_kend[3] = 1;
-            }
-        } else {
-            int Tk[kSplitTries];
-            Tk[0] = T0;
-#pragma unroll
-            for (int k = 1; k < kSplitTries; ++k) Tk[k] = Tk[k - 1] + Tk[k - 1] / 2;
-            auto pieces_of = [&](int kvl, int t) {
-                const int ub = kvl > 0 ? (kvl + kKvTile - 1) / kKvTile : 0;
-                return min(kMaxPieces, max(1, (2 * ub + t) / (2 * t)));
-            };
-            // pieces per KV head group for each T, then unsplit, then the
-            // sequences the decode workers run
-            int cnt[kSplitTries + 2] = {};
-            for (int base = 0; base < a.num_seqs; base += 256) {
-                const int i = base + tid;
-                int c[kSplitTries + 2] = {};
-                if (i < a.num_seqs) {
-                    int ql, kvl;
-                    seq_sizes(i, ql, kvl);
-                    const int nt = ql > 0 ? (ql + BT - 1) / BT : 0;
-#pragma unroll
-                    for (int k = 0; k < kSplitTries; ++k) c[k] = split ? nt * pieces_of(kvl, Tk[k]) : nt;
-                    c[kSplitTries] = nt;
-                    if constexpr (FUSED)
-                        c[kSplitTries + 1] = i < 256 ? my_dec : (a.cu_seqlens[i + 1] - a.cu_seqlens[i] == 1);
-                }
-                block_reduce_n(c, s_red);
-#pragma unroll
-                for (int k = 0; k <= kSplitTries + 1; ++k) cnt[k] += c[k];
-            }
-            if constexpr (FUSED) spread = __builtin_amdgcn_readfirstlane(cnt[kSplitTries + 1]) > 0;
-            int T = 0, total = cnt[kSplitTries];
+            if constexpr (FUSED) spread = __ballot(dec) != 0;
+            const int nt = ql > 0 ? (ql + BT - 1) / BT : 0;
+            int pp = 1, total = wave_sum_i32(nt);
             if (split) {
-#pragma unroll
-                for (int k = kSplitTries - 1; k >= 0; --k) {
-                    if ((int64_t)groups * cnt[k] <= a.resident) {
-                        T = Tk[k];
-                        total = cnt[k];
+                const int64_t all = (int64_t)wave_sum_i32(key_tiles(ql, kvl)) * groups;
+                int T = max(8, (int)((all + a.resident - 1) / a.resident));
+                split = false;
+                for (int k = 0; k < kSplitTries && !split; ++k, T += T / 2) {
+                    const int p = pieces_of(kvl, T);
+                    const int c = wave_sum_i32(nt * p);
+                    if ((int64_t)groups * c <= a.resident) {
+                        split = true;
+                        pp = p;
+                        total = c;
                     }
                 }
             }
-            split = T > 0;
             const int work = groups * total;
             const int per_xcd = (work + 7) >> 3;
             if ((lin >> 3) >= per_xcd) return;
@@ -413,50 +343,177 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             if (w >= work) return;
             grp = w / total;
             tile_lin = w - grp * total;
-
-            // The sequence of piece tile_lin.  Within a sequence come first the
-            // first pieces of all its query tiles (heaviest, i.e. last, tile
-            // first), then the second pieces, and so on: lengths fall smoothly
-            // along the dispatch order, so no run of long pieces queues behind
-            // one shader engine while others idle.
-            int carry = 0;
-            for (int base = 0; base < a.num_seqs; base += 256) {
-                const int i = base + tid;
-                int nt = 0, pp = 1, ql = 0, kvl = 0;
-                if (i < a.num_seqs) {
-                    seq_sizes(i, ql, kvl);
-                    nt = ql > 0 ? (ql + BT - 1) / BT : 0;
-                    pp = split ? pieces_of(kvl, T) : 1;
-                }
-                int tot;
-                const int incl = block_incl_scan(nt * pp, s_red, tot);
-                const int excl = incl - nt * pp;
-                if (i < a.num_seqs && tile_lin >= carry + excl && tile_lin < carry + incl) {
-                    s_seq = i;
-                    s_ltile = tile_lin - carry - excl;
-                    s_kend[0] = i < 256 ? my_q0 : a.cu_seqlens[i];  // q_begin (s_kend is rewritten below)
-                    s_kend[1] = ql;
-                    s_kend[2] = kvl;
-                    s_kend[3] = pp;
-                }
-                carry += tot;
-                if (carry > tile_lin) break;
+            const int incl = wave_incl_scan_i32(nt * pp);
+            const uint64_t here = __ballot(tile_lin < incl);
+            if (here == 0) return;
+            b = __builtin_ctzll(here);  // the first sequence that ends past the item
+            q_begin = __builtin_amdgcn_readlane(q0, b);
+            ql_b = __builtin_amdgcn_readlane(ql, b);
+            kv_len = __builtin_amdgcn_readlane(kvl, b);
+            npieces = __builtin_amdgcn_readlane(pp, b);
+            seq_tile = tile_lin - __builtin_amdgcn_readlane(incl - nt * pp, b);
+        } else {
+            // Per-sequence sizes, loaded once: thread t keeps sequence t (the
+            // passes below reload only for sequences past the first 256).
+            int my_q0 = 0, my_ql = 0, my_kvl = 0, my_dec = 0;
+            if (tid < a.num_seqs) {
+                my_q0 = a.cu_seqlens[tid];
+                my_ql = a.cu_seqlens[tid + 1] - my_q0;
+                my_dec = a.skip_decode_rows && my_ql == 1;
+                if (my_dec) my_ql = 0;  // run by the decode kernel
+                my_kvl = a.kv_lens[tid];
             }
+            auto seq_sizes = [&](int i, int& ql, int& kvl) {
+                if (i < 256) {
+                    ql = my_ql;
+                    kvl = my_kvl;
+                } else {
+                    ql = a.cu_seqlens[i + 1] - a.cu_seqlens[i];
+                    if (a.skip_decode_rows && ql == 1) ql = 0;
+                    kvl = a.kv_lens[i];
+                }
+            };
+            // Pieces per query tile of sequence i: round(key tiles / T), at most
+            // kMaxPieces, where T0 is the estimated key tiles per resident
+            // workgroup of the whole call.  A sequence up to 1.5 times the average
+            // is not split.
+            int T0 = 0;
+            if (split) {
+                for (int base = 0; base < a.num_seqs; base += 256) {
+                    const int i = base + tid;
+                    int est = 0;
+                    if (i < a.num_seqs) {
+                        int ql, kvl;
+                        seq_sizes(i, ql, kvl);
+                        est = key_tiles(ql, kvl);
+                    }
+                    int tot[1] = {est};
+                    block_reduce_n(tot, s_red);
+                    T0 += tot[0];
+                }
+                T0 = max(8, (int)(((int64_t)T0 * groups + a.resident - 1) / a.resident));
+            }
+            // Pieces only pay off in workgroup slots that would otherwise idle
+            // (a second round of pieces costs more than it balances): of the
+            // candidates T0, 1.5 T0, 2.25 T0, 3.375 T0 (fewer sequences split
+            // each time) the first whose pieces all fit in the resident slots at
+            // once is taken, else the call runs unsplit.
+            w = 0;
+            if (tid == 0) s_seq = -1;
+            if (!split && a.num_seqs <= 256) {
+                // Unsplit call, one sequence per thread: a single scan gives both
+                // the work total and each sequence's first query tile.
+                const int nt = tid < a.num_seqs && my_ql > 0 ? (my_ql + BT - 1) / BT : 0;
+                // beside decode workers with one-token sequences the copies are spread
+                if constexpr (FUSED) spread = __syncthreads_or(my_dec) != 0;
+                int total;
+                const int incl = block_incl_scan(nt, s_red, total);
+                const int work = groups * total;
+                const int per_xcd = (work + 7) >> 3;
+                if ((lin >> 3) >= per_xcd) return;
+                w = (lin & 7) * per_xcd + serpentine(lin >> 3, per_xcd, a.resident >> 4);
+                if (w >= work) return;
+                grp = w / total;
+                tile_lin = w - grp * total;
+                if (nt > 0 && tile_lin >= incl - nt && tile_lin < incl) {
+                    s_seq = tid;
+                    s_ltile = tile_lin - (incl - nt);
+                    s_kend[0] = my_q0;  // q_begin (s_kend is rewritten below)
+                    s_kend[1] = my_ql;
+                    s_kend[2] = my_kvl;
+                    s_kend[3] = 1;
+                }
+            } else {
+                int Tk[kSplitTries];
+                Tk[0] = T0;
+#pragma unroll
+                for (int k = 1; k < kSplitTries; ++k) Tk[k] = Tk[k - 1] + Tk[k - 1] / 2;
+                // pieces per KV head group for each T, then unsplit, then the
+                // sequences the decode workers run
+                int cnt[kSplitTries + 2] = {};
+                for (int base = 0; base < a.num_seqs; base += 256) {
+                    const int i = base + tid;
+                    int c[kSplitTries + 2] = {};
+                    if (i < a.num_seqs) {
+                        int ql, kvl;
+                        seq_sizes(i, ql, kvl);
+                        const int nt = ql > 0 ? (ql + BT - 1) / BT : 0;
+#pragma unroll
+                        for (int k = 0; k < kSplitTries; ++k) c[k] = split ? nt * pieces_of(kvl, Tk[k]) : nt;
+                        c[kSplitTries] = nt;
+                        if constexpr (FUSED)
+                            c[kSplitTries + 1] = i < 256 ? my_dec : (a.cu_seqlens[i + 1] - a.cu_seqlens[i] == 1);
+                    }
+                    block_reduce_n(c, s_red);
+#pragma unroll
+                    for (int k = 0; k <= kSplitTries + 1; ++k) cnt[k] += c[k];
+                }
+                if constexpr (FUSED) spread = __builtin_amdgcn_readfirstlane(cnt[kSplitTries + 1]) > 0;
+                int T = 0, total = cnt[kSplitTries];
+                if (split) {
+#pragma unroll
+                    for (int k = kSplitTries - 1; k >= 0; --k) {
+                        if ((int64_t)groups * cnt[k] <= a.resident) {
+                            T = Tk[k];
+                            total = cnt[k];
+                        }
+                    }
+                }
+                split = T > 0;
+                const int work = groups * total;
+                const int per_xcd = (work + 7) >> 3;
+                if ((lin >> 3) >= per_xcd) return;
+                w = (lin & 7) * per_xcd + (split ? (lin >> 3) : serpentine(lin >> 3, per_xcd, a.resident >> 4));
+                if (w >= work) return;
+                grp = w / total;
+                tile_lin = w - grp * total;
+
+                // The sequence of piece tile_lin.  Within a sequence come first the
+                // first pieces of all its query tiles (heaviest, i.e. last, tile
+                // first), then the second pieces, and so on: lengths fall smoothly
+                // along the dispatch order, so no run of long pieces queues behind
+                // one shader engine while others idle.
+                int carry = 0;
+                for (int base = 0; base < a.num_seqs; base += 256) {
+                    const int i = base + tid;
+                    int nt = 0, pp = 1, ql = 0, kvl = 0;
+                    if (i < a.num_seqs) {
+                        seq_sizes(i, ql, kvl);
+                        nt = ql > 0 ? (ql + BT - 1) / BT : 0;
+                        pp = split ? pieces_of(kvl, T) : 1;
+                    }
+                    int tot;
+                    const int incl = block_incl_scan(nt * pp, s_red, tot);
+                    const int excl = incl - nt * pp;
+                    if (i < a.num_seqs && tile_lin >= carry + excl && tile_lin < carry + incl) {
+                        s_seq = i;
+                        s_ltile = tile_lin - carry - excl;
+                        s_kend[0] = i < 256 ? my_q0 : a.cu_seqlens[i];  // q_begin (s_kend is rewritten below)
+                        s_kend[1] = ql;
+                        s_kend[2] = kvl;
+                        s_kend[3] = pp;
+                    }
+                    carry += tot;
+                    if (carry > tile_lin) break;
+                }
+            }
+            __syncthreads();
+            b = __builtin_amdgcn_readfirstlane(s_seq);
+            if (b < 0) return;
+            q_begin = __builtin_amdgcn_readfirstlane(s_kend[0]);
+            ql_b = __builtin_amdgcn_readfirstlane(s_kend[1]);
+            kv_len = __builtin_amdgcn_readfirstlane(s_kend[2]);
+            npieces = __builtin_amdgcn_readfirstlane(s_kend[3]);
+            seq_tile = __builtin_amdgcn_readfirstlane(s_ltile);
+            __syncthreads();  // s_kend is reused below
         }
-        __syncthreads();
-        b = s_seq;
-        if (b < 0) return;
-        q_begin = s_kend[0];
-        q_end = q_begin + s_kend[1];
-        kv_len = s_kend[2];
-        npieces = s_kend[3];
-        const int nt = (s_kend[1] + BT - 1) / BT;
-        piece = s_ltile / nt;
-        const int jh = s_ltile - piece * nt;
+        q_end = q_begin + ql_b;
+        const int nt = (ql_b + BT - 1) / BT;
+        piece = seq_tile / nt;
+        const int jh = seq_tile - piece * nt;
         tile = nt - 1 - jh;  // heaviest tile of the sequence first
-        sib_base = w - s_ltile + jh;
+        sib_base = w - seq_tile + jh;
         sib_stride = nt;
-        __syncthreads();  // s_kend is reused below
     } else {
         const int per_xcd = (int)gridDim.x >> 3;
         const int w = (lin & 7) * per_xcd + (lin >> 3);

@@ -310,3 +310,32 @@ def test_too_small_workspace_is_rejected(ops, gpu):
     rc = _C._lib.femto_paged_attention_gemm(*args, ws.data_ptr(), need, None)
     torch.cuda.synchronize()
     assert rc == 0 and int(torch.count_nonzero(ws)) == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads", [(16, 8), (32, 8), (3, 3)], ids=str)
+@pytest.mark.parametrize("seed", range(6))
+def test_work_list_of_few_and_many_sequences(ops, gpu, dtype, heads, seed):
+    """Up to 64 sequences each wave finds its work item by itself, above them the workgroup does it together.
+    The same batch alone (1 to 64 sequences, some empty, some of one token) and followed by empty sequences
+    (to 65 and to 300) agrees with the oracle, split calls, unsplit ones and ones with decode rows alike."""
+    rng = np.random.default_rng(seed)
+    n = [1, 2, 7, 33, 63, 64][seed]
+    big = 2500 if n <= 7 else 300
+    chunks = [(int(rng.integers(0, big)), int(rng.choice([0, 1, 2, 31, 64, 65, 200]))) for _ in range(n)]
+    chunks[0] = (chunks[0][0], 130)  # not all empty
+    w = workloads.make_paged_workload("work_list", chunks, *heads, seed=seed, dtype=dtype)
+    q, meta = w.gemm_call(device=gpu)
+    wd, q = w.to(gpu), q.to(gpu)
+    want = oa.paged_prefill(np64(q), np32(w.k_pool), np32(w.v_pool), meta.raw_cu_seqlens, np_tables(meta),
+                            meta.kv_lens.tolist(), np.asarray(meta.raw_positions))
+    for total in (n, 65, 300):
+        pad = total - n
+        cu = torch.cat([meta.cu_seqlens, meta.cu_seqlens[-1:].repeat(pad)])
+        kv = torch.cat([meta.kv_lens, meta.kv_lens.new_zeros(pad)])
+        tables = torch.cat([meta.block_tables, meta.block_tables.new_full((pad, meta.block_tables.size(1)), -1)])
+        out = ops.paged_attention_gemm(q, wd.k_pool, wd.v_pool, cu, meta.max_q_len, meta.Q_TILE_SIZE, meta.cu_q_tiles,
+                                       meta.q_tile_to_seq_idx, tables, kv, meta.positions)
+        torch.cuda.synchronize()
+        assert_close(out, want, dtype, f"work list {heads} {dtype} {n} of {total} sequences")
+    assert _workspace_is_zero(gpu)
