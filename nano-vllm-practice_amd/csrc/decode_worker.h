@@ -502,7 +502,7 @@ __device__ __forceinline__ void publish_and_merge(const DecodeArgs& a, int b, in
         u32x4v v[kU][NREP][2];
 #pragma unroll
         for (int u = 0; u < kU; ++u) {
-            const int i = min(i0 + 4 * u + rg, count - 1);  // past the end: the last slot again, with weight 0
+            const int i = min(i0 + 4 * u + rg, count - 1);  // past the end: the last slot again, left out below
 #pragma unroll
             for (int r = 0; r < NREP; ++r) {
                 const int sl = slot_of(r, i);
@@ -520,10 +520,11 @@ __device__ __forceinline__ void publish_and_merge(const DecodeArgs& a, int b, in
             for (int r = 0; r < NREP; ++r) {
                 const float ms = __uint_as_float(ml[u][r][0]);
                 const float mn = live ? fmaxf(M[r], ms) : M[r];
-                const float f0 = fast_exp2(M[r] - mn), f1 = live ? fast_exp2(ms - mn) : 0.0f;
-                L[r] = L[r] * f0 + __uint_as_float(ml[u][r][1]) * f1;
+                const float f0 = fast_exp2(M[r] - mn), f1 = fast_exp2(ms - mn);
+                L[r] = L[r] * f0 + (live ? __uint_as_float(ml[u][r][1]) * f1 : 0.0f);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) A[r][e] = A[r][e] * f0 + __uint_as_float(v[u][r][e >> 2][e & 3]) * f1;
+                for (int e = 0; e < 8; ++e)
+                    A[r][e] = A[r][e] * f0 + (live ? __uint_as_float(v[u][r][e >> 2][e & 3]) * f1 : 0.0f);
                 M[r] = mn;
             }
         }

@@ -57,3 +57,30 @@ def test_no_workspace_within_the_limit(gpu, dtype):
     torch.cuda.synchronize()
     want = oa.paged_decode(np64(q), np32(w.k_pool), np32(w.v_pool), np_tables(meta), meta.kv_lens.tolist())
     assert_close(out, want, dtype, "no workspace")
+
+
+@pytest.mark.parametrize("heads", [(16, 8), (16, 16)], ids=str)
+@pytest.mark.parametrize("keys", [1030, 1500, 2900])
+def test_infinite_values_stay_infinite(ops, gpu, heads, keys):
+    """Equal scores, and V infinite in the first key and in the last page of one dim each: both merges of split
+    contexts (the merge launch, and the one in a prefill call's launch) give infinities there and the mean of
+    V elsewhere, whatever the number of slots."""
+    w = workloads.make_paged_workload("inf", [(keys - 1, 1), (20, 9)], *heads, seed=61, poison=False)
+    q, meta = w.gemm_call(device=gpu)
+    wd = w.to(gpu)
+    wd.k_pool.zero_()
+    table = meta.block_tables[0].tolist()
+    wd.v_pool[table[0], :, 0, 3] = float("inf")
+    wd.v_pool[table[(keys - 1) // 16], :, 0, 5] = float("-inf")
+    q = q.to(gpu)
+    v = wd.v_pool[torch.tensor(table[: (keys + 15) // 16], device=gpu)].float().permute(1, 0, 2, 3).flatten(1, 2)[:, :keys]
+    want = v.mean(1).repeat_interleave(heads[0] // heads[1], 0)
+    rows = [ops.paged_attention_gemv(q[:, :1], wd.k_pool, wd.v_pool, meta.block_tables[:1], meta.kv_lens[:1], keys)[:, 0],
+            ops.paged_attention_gemm(q, wd.k_pool, wd.v_pool, meta.cu_seqlens, meta.max_q_len, meta.Q_TILE_SIZE,
+                                     meta.cu_q_tiles, meta.q_tile_to_seq_idx, meta.block_tables, meta.kv_lens,
+                                     meta.positions)[:, 0]]
+    for got in rows:
+        assert torch.isposinf(got[:, 3]).all() and torch.isneginf(got[:, 5]).all()
+        rest = [d for d in range(128) if d not in (3, 5)]
+        # probabilities 1/n rounded to bf16 cancel in the quotient; the output rounding is 2^-9 relative
+        assert torch.allclose(got[:, rest].float(), want[:, rest], rtol=2.0 ** -8, atol=1e-4)
