@@ -33,9 +33,10 @@
 //    without a look at the new scores: a row's maximum would have to wait
 //    for all of the tile's scores before the first exponential.  The row
 //    sum that the block needs anyway tells afterwards whether that was good
-//    enough (every P is at most the sum): above kMaxBlockSum, or infinite,
-//    the block's maximum is taken and its exponentials are redone before
-//    P.V reads them.  Inputs with a tile-by-tile rising maximum take that
+//    enough (every P is at most its growth): more than kMaxBlockSum, or
+//    infinite, and the block's maximum is taken and its exponentials are
+//    redone before P.V reads them.  The first tile has no running max and
+//    takes its maximum over both blocks.  Inputs with a tile-by-tile rising maximum take that
 //    path once per growth of the sum past 2^8.  Against a maximum per tile
 //    before the first exponential: 2048 x 8192 dense 252 -> 240 us, the last
 //    2048 tokens of a 32k prompt 963 -> 955 us, 8 x 512 73.3 -> 72.6 us, 4
@@ -74,7 +75,7 @@ constexpr int kStages = 2;
 constexpr int kRowBytes = kDimHead * 2;                // 256
 constexpr int kTileBytes = kKvTile * kRowBytes;        // 16 KB per K or V tile
 constexpr float kEmptyMaxP = -1.0e30f;
-constexpr float kMaxBlockSum = 256.0f;  // largest sum of a row's 16 exponentials in a lane before the running max moves
+constexpr float kMaxBlockSum = 256.0f;  // largest growth of a lane's row sum in a block (16 exponentials) before the running max moves
 constexpr int kSplitTries = 4;  // key-split granularities tried (T grows by half each time)
 
 // One page of zeros: the source of every copy whose block id lies outside
@@ -717,8 +718,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const float scale = a.scale_log2;
 
     // One 64-key tile from LDS stage STAGE (a compile-time constant, so the
-    // stage offset folds into the LDS instructions' immediate offsets).
-    auto tile_math = [&](int kb, auto stage_c, auto copies_c) __attribute__((always_inline)) {
+    // stage offset folds into the LDS instructions' immediate offsets);
+    // first: the piece's first tile, no row has a running max yet.
+    auto tile_math = [&](int kb, bool first, auto stage_c, auto copies_c) __attribute__((always_inline)) {
         constexpr int STAGE = decltype(stage_c)::value;
         // copies_c: std::false_type (no copies here), or a bool: issue the
         // next tile's copies between the score MFMAs
@@ -743,8 +745,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             }
             return u32x4{part[0][0], part[0][1], part[1][0], part[1][1]};
         };
-        // Values 2i and 2i + 1 of score block kb2 become two exponentials, one
-        // packed word of P and a term of the block's row sum.
+        // Values 2i and 2i + 1 of a score block become two exponentials, one
+        // packed word of P and a term of the row sum, which runs on from
+        // l_run: one chain over all of the lane's keys.
         float neg_m = -m_run;
         auto soft = [&](const f32x16& sv, int i, u32x4 (&pw)[2], float& sum) __attribute__((always_inline)) {
             float e[2];
@@ -756,10 +759,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             pw[i >> 2][i & 3] = w;
             sum = sum2(E{}, w, sum);
         };
+        f32x16 s0 = f32x16{}, s1 = f32x16{};
         // Before P.V reads a block's P: the mask, on tiles that cross a limit,
-        // and where some row's block sum passed kMaxBlockSum (out of line: it
-        // is rare) the running max moves to the block's and the exponentials
-        // are redone.
+        // and where some row's sum grew by more than kMaxBlockSum in the block
+        // (out of line: it is rare) the running max moves to the block's and
+        // the exponentials are redone.  A piece's first tile takes the maximum
+        // over both blocks (block 1's scores are there by then): over block 0
+        // alone the largest P of a row of up to 64 keys would often be rounded
+        // and not 1, which cost 1 % of accuracy on short prompts.  It has its
+        // own branch because the out-of-line one, reading s1 too, made the
+        // compiler copy or spill the accumulators on every tile.
         auto settle = [&](f32x16& sv, int kb2, u32x4 (&pw)[2], float& sum) __attribute__((always_inline)) {
             if (kb + kKvTile > kfull_w) {  // wave-uniform: the tile crosses some row's limit
 #pragma unroll
@@ -767,15 +776,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                     const int rel = 32 * kb2 + 8 * (x >> 2) + (x & 3);
                     sv[x] = rel < kr ? sv[x] : -INFINITY;
                 }
-                sum = 0.0f;
+                sum = l_run;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) soft(sv, i, pw, sum);
             }
-            if (__builtin_expect(__ballot(sum > kMaxBlockSum) != 0, 0)) {
+            if (kb2 == 0 && first) {
+                float mx = -INFINITY;
+#pragma unroll
+                for (int x = 0; x < 16; ++x) mx = fmaxf(mx, fmaxf(sv[x], 32 + 8 * (x >> 2) + (x & 3) < kr ? s1[x] : -INFINITY));
+                float m_lo, m_hi;  // the row's two lane halves (keys 4*h2 + ...)
+                pair32(mx, m_lo, m_hi);
+                m_run = fmaxf(m_run, fmaxf(m_lo, m_hi) * scale);
+                neg_m = -m_run;
+                sum = l_run;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) soft(sv, i, pw, sum);
+            }
+            if (__builtin_expect(__ballot(sum - l_run > kMaxBlockSum) != 0, 0)) {
                 float mx = sv[0];
 #pragma unroll
                 for (int x = 1; x < 16; ++x) mx = fmaxf(mx, sv[x]);
-                float m_lo, m_hi;  // the row's two lane halves (keys 4*h2 + ...)
+                float m_lo, m_hi;
                 pair32(mx, m_lo, m_hi);
                 const float m_new = fmaxf(m_run, fmaxf(m_lo, m_hi) * scale);
                 const float alpha = fast_exp2(m_run - m_new);
@@ -784,16 +805,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 l_run *= alpha;
 #pragma unroll
                 for (int dt = 0; dt < 4; ++dt) oacc[dt] *= alpha;
-                sum = 0.0f;
+                sum = l_run;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) soft(sv, i, pw, sum);
             }
-            l_run += sum;
+            l_run = sum;
         };
         constexpr int kAhead = 4;  // fragments read ahead of their MFMA (3: 1 % slower on long context)
-        f32x16 s0 = f32x16{}, s1 = f32x16{};
         u32x4 p0[2], p1[2];
-        float sum0 = 0.0f, sum1 = 0.0f;
+        float sum0 = l_run;
         u32x4 kf[kAhead + 1], vf[kAhead + 1];
         // Each MFMA is fenced into one bundle with the fragment read ahead of
         // it and its share of the other block's softmax: the compiler's own
@@ -825,6 +845,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         // (keeps the exponentials above from being sunk below settle's branches)
         asm volatile("" : "+v"(p0[0]), "+v"(p0[1]), "+v"(sum0));
         settle(s0, 0, p0, sum0);
+        float sum1 = l_run;
 #pragma unroll
         for (int n = 0; n < 8; ++n) {
             vf[(n + kAhead) % (kAhead + 1)] = vfrag(n + kAhead);
@@ -872,13 +893,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         const int kb = it * kKvTile;
         if constexpr (SPREAD) {
             if (kb < kend_w) {
-                tile_math(kb, stage_c, more);
+                tile_math(kb, STAGE == 0 && it == t_lo, stage_c, more);
             } else if (more) {
 #pragma unroll
                 for (int j = 0; j < 8; ++j) copy_one(j);
             }
         } else {
-            if (kb < kend_w) tile_math(kb, stage_c, std::false_type{});
+            if (kb < kend_w) tile_math(kb, STAGE == 0 && it == t_lo, stage_c, std::false_type{});
         }
     };
     auto tile_loop = [&](auto spread_c) __attribute__((always_inline)) {
