@@ -100,13 +100,15 @@ int femto_paged_attention_gemv(
  * sequences x 32 heads); larger calls fail with FEMTO_ERR_INVALID.  When the default
  * split does not fit the array, sequences are cut into fewer, longer slices
  * (same results within rounding; bit-identical where the split is the
- * same).  All calls on one GPU share the array: calls that may overlap on
- * one GPU (different streams or threads) race and must be serialised by the
- * caller.  The first call on a device looks up the array's device address and
- * the CU count (hipGetSymbolAddress, hipDeviceGetAttribute): make it outside
- * graph capture; later calls only launch kernels and may be captured.  Every
- * process that loads the library reserves the 64 MiB on each GPU it uses,
- * whether or not it calls this entry point. */
+ * same).  Calls within the one-launch limit (default 1024 keys) never use the
+ * array, whatever their shape.  All longer calls on one GPU share it: those
+ * that may overlap on one GPU (different streams or threads) race and must be
+ * serialised by the caller.  The first longer call on a device looks up the
+ * array's device address and the CU count (hipGetSymbolAddress,
+ * hipDeviceGetAttribute): make it outside graph capture; later calls only
+ * launch kernels and may be captured.  Every process that loads the library
+ * reserves the 64 MiB on each GPU it uses, whether or not it calls this entry
+ * point. */
 int femto_paged_attention_gemv_noalloc(
     int dtype,
     const void* q, int64_t q_stride_head, int64_t q_stride_seq,

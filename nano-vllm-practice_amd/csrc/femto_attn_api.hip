@@ -303,11 +303,13 @@ static int paged_decode_entry(const char* fn_name, int dtype, const void* q, int
     const femto::DecodeRoute route = femto::decode_route(num_seqs, n_heads, plan.nrep_tile, max_kv_len, dtype);
     const int limit = g_single_max_kv.load(std::memory_order_relaxed);
     bool single = max_kv_len <= limit;
-    if (single && limit == kSingleMaxKV && max_kv_len > route.max_kv) {
-        // The split route, if its partial slots fit: calls within the limit
-        // need no workspace, and no scratch.
+    if (single && !use_scratch && limit == kSingleMaxKV && max_kv_len > route.max_kv) {
+        // The split route, if the caller's workspace holds its partial slots:
+        // calls within the limit need none.  Never with the scratch: calls
+        // within the limit share no memory, so they may overlap on one GPU,
+        // and the first of them under graph capture looks up no address.
         const size_t slots = femto::decode_workspace_bytes(num_seqs, n_heads, plan.max_slots);
-        single = use_scratch ? slots > kScratchBytes : !workspace || workspace_bytes < slots || !aligned(workspace, 256);
+        single = !workspace || workspace_bytes < slots || !aligned(workspace, 256);
     }
     if (single) {
         // One launch, no workspace.  A max_kv_len below the true longest

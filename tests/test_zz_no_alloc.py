@@ -155,3 +155,34 @@ def test_noalloc_under_graph_capture(gpu, lens):
         assert torch.equal(out, eager), f"replay {rep}: graph output differs from the eager call"
         want = oa.paged_decode(np64(q_new), np32(w.k_pool), np32(w.v_pool), np_tables(meta), new_lens)
         assert_close(out, want, w.dtype, f"graph replay {rep}, lens {new_lens}")
+
+
+@pytest.mark.parametrize("heads,seqs", [((64, 8), 193), ((4, 4), 400), ((16, 8), 8)], ids=str)
+def test_noalloc_within_the_limit_is_one_launch(gpu, heads, seqs):
+    """f32 shapes that the workspace entry point runs split within 1024 keys: without a workspace they stay
+    on the one launch, which touches no memory that another call could share, so calls on two streams may
+    overlap and the first call may be captured.  The two routes sum in different orders, so equal bits tell
+    the route."""
+    from femtovllm import _C
+
+    lens = [int(x) for x in np.random.default_rng(seqs).integers(600, 1000, size=seqs)]
+    lens[0] = 1000
+    w = workloads.make_paged_workload("short", [(n - 1, 1) for n in lens], *heads, seed=seqs, dtype=torch.float32)
+    q, wd, meta = case(w, gpu)
+    args = (_C, q, wd.k_pool, wd.v_pool, meta.block_tables, meta.kv_lens, meta.max_kv_len)
+    prev = _C._lib.femto_attn_set_decode_single_max_kv(1 << 30)
+    try:
+        want = gemv_noalloc(*args)[1]
+    finally:
+        _C._lib.femto_attn_set_decode_single_max_kv(prev)
+    assert not torch.equal(gemv_with_workspace(*args), want), "the workspace call is meant to run split"
+    assert torch.equal(gemv_noalloc(*args)[1], want)
+    out = torch.full_like(q, float("nan"))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        gemv_noalloc(*args, out=out)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
