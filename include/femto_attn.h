@@ -60,9 +60,10 @@ size_t femto_paged_attention_gemv_workspace_size(int num_seqs, int n_heads, int 
  * one kernel launch (a workgroup per sequence and KV head group) and use no
  * workspace; longer ones run the split kernel and the merge kernel.  At the
  * default, shapes that run faster split whatever the lengths (large batches
- * with eight query heads per KV head or in f32) do so where a workspace is
- * given.  Sets the
- * limit for the process (-1: always split) and returns the previous one.
+ * with eight query heads per KV head or in f32, and a few f32 sequences near
+ * the limit) do so where a workspace is given, except under graph capture: a
+ * captured call within the limit holds no workspace.  Sets the limit for the
+ * process (-1: always split) and returns the previous one.
  * No counterpart in the reference (whose decode is always one launch,
  * csrc/paged_attention/paged_attention_gemv.cu:280-300); it exists for tests
  * and tuning. */

@@ -278,6 +278,15 @@ int decode_rows_bound(int num_seqs, int num_tokens, int max_q_len) {
 
 }  // namespace femto
 
+// Whether a launch on the stream would be recorded into a graph (or the stream
+// does not say, as the legacy stream while another thread captures).
+static bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 // Decode entry points: femto_paged_attention_gemv (workspace from the caller)
 // and femto_paged_attention_gemv_noalloc (workspace = this device's scratch).
 static int paged_decode_entry(const char* fn_name, int dtype, const void* q, int64_t q_stride_head,
@@ -308,8 +317,12 @@ static int paged_decode_entry(const char* fn_name, int dtype, const void* q, int
         // calls within the limit need none.  Never with the scratch: calls
         // within the limit share no memory, so they may overlap on one GPU,
         // and the first of them under graph capture looks up no address.
+        // Nor in a captured call: a graph that held the workspace would write
+        // it at every replay, beside other graphs and streams that the caller
+        // may run at the time and past the life of the memory.
         const size_t slots = femto::decode_workspace_bytes(num_seqs, n_heads, plan.max_slots);
-        single = !workspace || workspace_bytes < slots || !aligned(workspace, 256);
+        single = !workspace || workspace_bytes < slots || !aligned(workspace, 256) ||
+                 capturing(static_cast<hipStream_t>(stream));
     }
     if (single) {
         // One launch, no workspace.  A max_kv_len below the true longest

@@ -84,3 +84,51 @@ def test_infinite_values_stay_infinite(ops, gpu, heads, keys):
         rest = [d for d in range(128) if d not in (3, 5)]
         # probabilities 1/n rounded to bf16 cancel in the quotient; the output rounding is 2^-9 relative
         assert torch.allclose(got[:, rest].float(), want[:, rest], rtol=2.0 ** -8, atol=1e-4)
+
+
+@pytest.mark.parametrize("shape", [((64, 8), 193), ((16, 8), 8), ((4, 4), 400)], ids=str)
+def test_captured_call_within_the_limit_holds_no_workspace(ops, gpu, shape):
+    """f32 shapes that run split within 1024 keys: captured in a graph they are one launch (the routes sum in
+    different orders, so equal bits tell which one ran), and replays still match after the stream's workspace
+    was replaced by a larger one and its memory taken by another tensor."""
+    from femtovllm import _C
+
+    (heads, kv_heads), seqs = shape
+    lens = [int(x) for x in np.random.default_rng(seqs).integers(600, 1000, size=seqs)]
+    lens[0] = 1000
+    w = workloads.make_paged_workload("capture", [(n - 1, 1) for n in lens], heads, kv_heads, seed=seqs,
+                                      dtype=torch.float32)
+    q, meta = w.gemv_call(device=gpu)
+    wd, q = w.to(gpu), q.to(gpu).contiguous()
+    call = lambda: ops.paged_attention_gemv(q, wd.k_pool, wd.v_pool, meta.block_tables, meta.kv_lens, meta.max_kv_len)
+
+    def forced(limit):
+        prev = _C._lib.femto_attn_set_decode_single_max_kv(limit)
+        try:
+            return call()
+        finally:
+            _C._lib.femto_attn_set_decode_single_max_kv(prev)
+
+    one, split = forced(1 << 30), forced(-1)
+    assert not torch.equal(one, split) and torch.equal(call(), split)
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call()  # this stream's workspace
+        side.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            out = call()
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, one)
+    old = _C._workspaces[(gpu.index, side.cuda_stream)]
+    size = old.numel()
+    with torch.cuda.stream(side):
+        _C._decode_workspace(gpu, 2 * seqs, heads, 8192)
+        del old
+        other = torch.full((size,), 77, dtype=torch.uint8, device=gpu)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, one) and bool((other == 77).all())
