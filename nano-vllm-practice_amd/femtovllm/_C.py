@@ -149,6 +149,12 @@ def _dtype_code(t: torch.Tensor, fn: str) -> int:
 # one stream are ordered, so they can share it.
 _workspaces: dict = {}
 
+# Workspaces that a larger one replaced.  A graph captured while one was in
+# use writes it at every replay, so its memory must not go back to the
+# allocator.  Each replacement is at least twice as large, so all of these
+# together are smaller than the one in use.
+_replaced_workspaces: list = []
+
 
 def _cached_workspace(cache: dict, device: torch.device, nbytes: int, zero: bool):
     if nbytes == 0:
@@ -156,8 +162,12 @@ def _cached_workspace(cache: dict, device: torch.device, nbytes: int, zero: bool
     key = (device.index, _stream(device))
     ws = cache.get(key)
     if ws is None or ws.numel() < nbytes + 256:
+        size = nbytes + 256
+        if ws is not None:
+            size = max(size, 2 * ws.numel())
+            _replaced_workspaces.append(ws)
         alloc = torch.zeros if zero else torch.empty
-        ws = alloc(nbytes + 256, dtype=torch.uint8, device=device)
+        ws = alloc(size, dtype=torch.uint8, device=device)
         cache[key] = ws
     ptr = ws.data_ptr()
     aligned = (ptr + 255) & ~255
