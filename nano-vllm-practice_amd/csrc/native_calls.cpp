@@ -119,12 +119,25 @@ void check_paged(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, 
     need(k.size(1) > 0 && q.size(0) % k.size(1) == 0);
 }
 
-PyObject* finish(int rc, const at::Tensor& out) {
-    if (rc != 0) {
-        PyErr_SetString(PyExc_RuntimeError, g_last_error());
-        return nullptr;
+// The library call and its result.  The result's Python object is made first and whatever the library
+// throws is an error: nothing can decline the call once the library has been entered (the Python path
+// would make it a second time, on a q that the first may have overwritten).
+template <typename F>
+PyObject* launch(const at::Tensor& out, F call) {
+    PyObject* result = THPVariable_Wrap(out);
+    need(result != nullptr);
+    int rc;
+    PyThreadState* gil = PyEval_SaveThread();
+    try {
+        rc = call();
+    } catch (...) {
+        rc = -1;
     }
-    return THPVariable_Wrap(out);
+    PyEval_RestoreThread(gil);
+    if (rc == 0) return result;
+    Py_DECREF(result);
+    PyErr_SetString(PyExc_RuntimeError, rc < 0 ? "femto_native: the library threw" : g_last_error());
+    return nullptr;
 }
 
 template <typename F>
@@ -135,6 +148,7 @@ PyObject* guarded(Py_ssize_t n, Py_ssize_t want, F f) {
     } catch (const NotHere&) {
     } catch (const std::exception&) {  // raised again, as Python sees it, by the Python path
     }
+    PyErr_Clear();
     Py_RETURN_NONE;
 }
 
@@ -154,13 +168,11 @@ PyObject* gemv(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const void *qp = q.const_data_ptr(), *kp = k.const_data_ptr(), *vp = v.const_data_ptr();
         const int32_t *tp = i32(tab), *lp = i32(len);
         void* op = out.data_ptr();
-        int rc;
-        Py_BEGIN_ALLOW_THREADS
-        rc = g_gemv(dt, qp, q.stride(0), q.stride(1), op, out.stride(0), out.stride(1), kp, vp, k.size(0), (int)k.size(1),
-                    (int)k.size(2), (int)k.size(3), k.stride(0), k.stride(1), k.stride(2), tp, (int)tab.size(1),
-                    tab.stride(0), lp, (int)B, (int)H, max_kv, w.ptr, w.bytes, st);
-        Py_END_ALLOW_THREADS
-        return finish(rc, out);
+        return launch(out, [&] {
+            return g_gemv(dt, qp, q.stride(0), q.stride(1), op, out.stride(0), out.stride(1), kp, vp, k.size(0), (int)k.size(1),
+                          (int)k.size(2), (int)k.size(3), k.stride(0), k.stride(1), k.stride(2), tp, (int)tab.size(1),
+                          tab.stride(0), lp, (int)B, (int)H, max_kv, w.ptr, w.bytes, st);
+        });
     });
 }
 
@@ -184,13 +196,11 @@ PyObject* gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const void *qp = q.const_data_ptr(), *kp = k.const_data_ptr(), *vp = v.const_data_ptr();
         const int32_t *cp = i32(cu), *tp = i32(tab), *lp = i32(len), *pp = i32(pos);
         void* op = out.data_ptr();
-        int rc;
-        Py_BEGIN_ALLOW_THREADS
-        rc = g_gemm(dt, qp, q.stride(0), q.stride(1), op, out.stride(0), out.stride(1), kp, vp, k.size(0), (int)k.size(1),
-                    (int)k.size(2), (int)k.size(3), k.stride(0), k.stride(1), k.stride(2), cp, (int)B, (int)T, max_q, (int)H,
-                    tp, (int)tab.size(1), tab.stride(0), lp, pp, w.ptr, w.bytes, st);
-        Py_END_ALLOW_THREADS
-        return finish(rc, out);
+        return launch(out, [&] {
+            return g_gemm(dt, qp, q.stride(0), q.stride(1), op, out.stride(0), out.stride(1), kp, vp, k.size(0), (int)k.size(1),
+                          (int)k.size(2), (int)k.size(3), k.stride(0), k.stride(1), k.stride(2), cp, (int)B, (int)T, max_q, (int)H,
+                          tp, (int)tab.size(1), tab.stride(0), lp, pp, w.ptr, w.bytes, st);
+        });
     });
 }
 
@@ -241,14 +251,12 @@ PyObject* prologue(PyObject*, PyObject* const* a, Py_ssize_t n) {
         void *od = out.data_ptr(), *kpd = kp.data_ptr(), *vpd = vp.data_ptr();
         const int32_t *pd = i32(pos), *td = i32(tab);
         const int H = int32(q.size(1)), rows = int32(cos.size(0)), tokens = int32(T), seqs = int32(B);
-        int rc;
-        Py_BEGIN_ALLOW_THREADS
-        rc = g_prologue(dt, qd, q.stride(0), q.stride(1), kd, k.stride(0), k.stride(1), vd, v.stride(0), v.stride(1), od,
-                        out.stride(0), out.stride(1), wqd, wkd, eps, cd, sd, cos.stride(0), rows, kpd, vpd, kp.size(0), H,
-                        (int)kp.size(1), (int)kp.size(2), (int)kp.size(3), kp.stride(0), kp.stride(1), kp.stride(2), cp, seqs,
-                        tokens, max_q, pd, td, (int)tab.size(1), tab.stride(0), st);
-        Py_END_ALLOW_THREADS
-        return finish(rc, out);
+        return launch(out, [&] {
+            return g_prologue(dt, qd, q.stride(0), q.stride(1), kd, k.stride(0), k.stride(1), vd, v.stride(0), v.stride(1), od,
+                              out.stride(0), out.stride(1), wqd, wkd, eps, cd, sd, cos.stride(0), rows, kpd, vpd, kp.size(0), H,
+                              (int)kp.size(1), (int)kp.size(2), (int)kp.size(3), kp.stride(0), kp.stride(1), kp.stride(2), cp, seqs,
+                              tokens, max_q, pd, td, (int)tab.size(1), tab.stride(0), st);
+        });
     });
 }
 
@@ -268,13 +276,11 @@ PyObject* flash(PyObject*, PyObject* const* a, Py_ssize_t n) {
         void* op = out.data_ptr();
         const int B = int32(q.size(0)), H = int32(q.size(1)), KVH = int32(k.size(1)), Tq = int32(q.size(2)),
                   Tk = int32(k.size(2));
-        int rc;
-        Py_BEGIN_ALLOW_THREADS
-        rc = g_flash(dt, qp, q.stride(0), q.stride(1), q.stride(2), kp, k.stride(0), k.stride(1), k.stride(2), vp,
-                     v.stride(0), v.stride(1), v.stride(2), op, out.stride(0), out.stride(1), out.stride(2), B, H, KVH, Tq,
-                     Tk, 128, st);
-        Py_END_ALLOW_THREADS
-        return finish(rc, out);
+        return launch(out, [&] {
+            return g_flash(dt, qp, q.stride(0), q.stride(1), q.stride(2), kp, k.stride(0), k.stride(1), k.stride(2), vp,
+                           v.stride(0), v.stride(1), v.stride(2), op, out.stride(0), out.stride(1), out.stride(2), B, H, KVH, Tq,
+                           Tk, 128, st);
+        });
     });
 }
 
