@@ -193,7 +193,10 @@ def _prefill_workspace(device: torch.device, num_seqs: int, num_tokens: int, max
     return _cached_workspace(_prefill_workspaces, device, nbytes, zero=True)
 
 
-_stream_prefill_workspace = _prefill_workspace  # a caller that replaces _prefill_workspace gets the Python path
+# The native calls look the workspaces up by themselves: a caller that replaces one of the functions
+# above gets the Python path, which asks it.
+_stream_decode_workspace = _decode_workspace
+_stream_prefill_workspace = _prefill_workspace
 
 
 def _check_paged(fn, q, k_pool, v_pool, tables, kv_lens, require_contiguous_q, decode=False):
@@ -232,10 +235,11 @@ def _paged_attention_gemv(q, k_pool, v_pool, kv_page_tables, kv_lens, max_kv_len
     """Decode through the C ABI.  ``max_kv_len_limit`` is the reference's
     ``kMaxKVLenNonSplit`` check (paged_attention_gemv.cu:271-274); ``None``
     lifts it, since the kernel splits contexts of any length over waves."""
-    out = _native.gemv(q, k_pool, v_pool, kv_page_tables, kv_lens, max_kv_len, require_contiguous_q,
-                       max_kv_len_limit, _workspaces)
-    if out is not None:
-        return out
+    if _decode_workspace is _stream_decode_workspace:
+        out = _native.gemv(q, k_pool, v_pool, kv_page_tables, kv_lens, max_kv_len, require_contiguous_q,
+                           max_kv_len_limit, _workspaces)
+        if out is not None:
+            return out
     fn = "PagedAttentionGemvCuda"
     _check_paged(fn, q, k_pool, v_pool, kv_page_tables, kv_lens, require_contiguous_q, decode=True)
     n_heads, num_seqs, dim = q.shape

@@ -36,6 +36,31 @@ def test_replaced_workspaces_stay_allocated_and_bounded(monkeypatch):
     assert sum(r().numel() for r in seen[:-1]) < seen[-1]().numel()
 
 
+@pytest.mark.parametrize("name,function", [("gemv", "_decode_workspace"), ("gemm", "_prefill_workspace")])
+def test_a_replaced_workspace_function_is_asked(monkeypatch, name, function):
+    """The native call looks the stream's workspace up by itself, so it is left out once the function is not
+    the module's own."""
+    from femtovllm import _C
+
+    asked = []
+
+    class Native:
+        def __getattr__(self, entry):
+            return lambda *args: asked.append(entry)
+
+    q, pool, i32 = torch.zeros(2, 1, 128), torch.zeros(1, 1, 16, 128), torch.zeros(1, dtype=torch.int32)
+    call = {"gemv": lambda: _C.PagedAttentionGemvCuda(q, pool, pool, i32[None], i32, 1),
+            "gemm": lambda: _C.PagedAttentionGemmCuda(q, pool, pool, i32, 1, i32[None], i32, i32)}[name]
+    monkeypatch.setattr(_C, "_native", Native())
+    with pytest.raises(RuntimeError, match="GPU tensor"):
+        call()
+    assert asked == [name]
+    monkeypatch.setattr(_C, function, lambda *args: (None, 0))
+    with pytest.raises(RuntimeError, match="GPU tensor"):
+        call()
+    assert asked == [name]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("entry", ["decode", "prefill"])
 def test_replay_after_the_workspace_grew(ops, gpu, entry):
