@@ -13,6 +13,7 @@
 #include <string>
 
 #include "common.h"
+#include "decode_route.h"
 #include "femto_attn.h"
 #include "launch.h"
 
@@ -26,8 +27,8 @@ thread_local std::string g_err;
 
 // Decode calls whose max_kv_len is at most this run as one launch (a
 // workgroup per sequence and KV head group, no workspace); longer ones use
-// the split workers and the merge kernel.  At the default decode_route may
-// lower it for the call's shape; any other value is taken as it is.
+// the split workers and the merge kernel.  At the default decode_route sends
+// some shapes there within it; any other value is taken as it is.
 constexpr int kSingleMaxKV = 1024;
 std::atomic<int> g_single_max_kv{kSingleMaxKV};
 
@@ -171,56 +172,6 @@ size_t decode_workspace_bytes(int num_seqs, int n_heads, int max_slots) {
     return bytes + (size_t)num_seqs * sizeof(int);
 }
 
-// Form of a one-launch decode call, and up to which max_kv_len it is taken
-// rather than the split workers and their merge launch.
-struct DecodeRoute {
-    int nrep_tile, waves, max_kv;
-};
-
-// The one-launch kernel takes whole sequences: a call ends with its longest
-// sequence and with the CU that got the most workgroups, but needs no merge
-// launch (~4 us).  The host knows the longest context only, so the split route
-// is taken below 1024 keys only where it won over batches of equal lengths and
-// of lengths spread over a factor of eight alike (2-256 sequences, 32-1024
-// keys, five head shapes, each form of both routes; us per call, spread
-// lengths where not said):
-//  * 16-bit types, at most one workgroup per CU (256): as few query heads per
-//    wave as keep the call there, and eight waves, so a wave walks half the
-//    pages: 16 sequences up to 1024 keys on 32/8 heads 22.2 (four heads, four
-//    waves) -> 16.3 (two heads, eight waves; split 20.7), 8 on 64/8 heads 32.3
-//    (eight heads) -> 14.9.  Four heads fill the registers of a CU with four
-//    waves already; eight of them pay off above 512 keys only (16 sequences on
-//    64/8 heads 22.2 -> 20.9 at 1024 keys, 13.7 -> 13.8 at 512);
-//  * more workgroups: four waves of all (at most four) heads;
-//  * eight heads per wave need over 256 registers, one wave per SIMD; two
-//    workgroups of four heads read the pages twice but are faster up to 512
-//    keys (64 equal sequences of 128 keys: 20.6 -> 16.3) and, in rounds of
-//    workgroups, up to 256 (128 sequences: 49.3 -> 39.9; 512 keys: 73.2, split
-//    53.0, equal lengths 80.0 and 74.2).  With 256 sequences the split route
-//    is always ahead (32 equal keys: 52.2 -> 29.5);
-//  * f32 (twice the bytes and registers per page): one head and eight waves up
-//    to 256 (sequence, head) pairs; half the CUs idle lose to the split route
-//    near 1024 keys (8 sequences on 16/8 heads: 22.7, split 18.0), and with 256
-//    sequences on 16/8 heads it is always ahead (equal 128 keys: 57.4, 49.7).
-static DecodeRoute decode_route(int num_seqs, int n_heads, int plan_nrep, int max_kv_len, int dtype) {
-    const int64_t pairs = (int64_t)num_seqs * n_heads;
-    constexpr int kCUs = 256;
-    if (dtype == kDtypeF32) {
-        if (pairs <= kCUs) return {1, 8, pairs <= kCUs / 2 ? 896 : 1024};
-        return {plan_nrep, 4, pairs / plan_nrep > 6 * kCUs ? 0 : 1024};
-    }
-    const int most = std::min(plan_nrep, 4);
-    int r = 1;
-    while (r < most && pairs / r > kCUs) r *= 2;
-    const int64_t groups = pairs / r;
-    if (groups <= kCUs) return {r, r == 4 && max_kv_len <= 512 ? 4 : 8, 1024};
-    if (plan_nrep == 8) {
-        if (groups > 4 * kCUs) return {4, 4, groups > 12 * kCUs ? 0 : 256};
-        if (max_kv_len > 512) return {8, 4, 1024};
-    }
-    return {r, 4, 1024};
-}
-
 // Kernel arguments of a decode launch over the pools; q rows / out rows b
 // (decode call) or cu_seqlens[b] (decode rows of a prefill call).
 DecodeArgs decode_args(const DecodePlan& plan, const void* q, int64_t q_stride_head, int64_t q_stride_row, void* out,
@@ -309,10 +260,16 @@ static int paged_decode_entry(const char* fn_name, int dtype, const void* q, int
     if (rc != FEMTO_OK) return rc;
 
     femto::DecodePlan plan = femto::plan_paged_decode(n_heads, n_kv_heads, max_kv_len, dtype);
-    const femto::DecodeRoute route = femto::decode_route(num_seqs, n_heads, plan.nrep_tile, max_kv_len, dtype);
     const int limit = g_single_max_kv.load(std::memory_order_relaxed);
     bool single = max_kv_len <= limit;
-    if (single && !use_scratch && limit == kSingleMaxKV && max_kv_len > route.max_kv) {
+    femto::DecodeRoute route{};
+    if (single) {
+        int cus = 0;
+        rc = hip_status(femto::device_cu_count(cus), (fn + ": device query").c_str());
+        if (rc != FEMTO_OK) return rc;
+        route = femto::decode_route(num_seqs, n_heads, n_kv_heads, plan.nrep_tile, max_kv_len, dtype == FEMTO_F32, cus);
+    }
+    if (single && route.split && !use_scratch && limit == kSingleMaxKV) {
         // The split route, if the caller's workspace holds its partial slots:
         // calls within the limit need none.  Never with the scratch: calls
         // within the limit share no memory, so they may overlap on one GPU,

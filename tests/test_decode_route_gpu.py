@@ -39,6 +39,21 @@ def test_route_edges(ops, gpu, dtype, longest, shape):
     assert_close(out, want, dtype, f"decode route {shape} {longest} {dtype}")
 
 
+# (heads, kv_heads, sequences, longest): on both sides of the lines by key count, rounds and head ratio
+LINES = [(8, 1, 137, 128), (8, 1, 137, 129), (64, 8, 34, 512), (64, 8, 34, 513), (64, 8, 65, 257), (24, 2, 21, 768),
+         (24, 2, 21, 769), (16, 8, 24, 500), (16, 8, 25, 500), (2, 1, 256, 1000)]
+
+
+@pytest.mark.parametrize("shape", LINES, ids=str)
+def test_route_lines(ops, gpu, shape):
+    w = _batch(*shape, torch.bfloat16)
+    q, meta = w.gemv_call(device=gpu)
+    wd = w.to(gpu)
+    out = ops.paged_attention_gemv(q.to(gpu), wd.k_pool, wd.v_pool, meta.block_tables, meta.kv_lens, meta.max_kv_len)
+    want = oa.paged_decode(np64(q), np32(w.k_pool), np32(w.v_pool), np_tables(meta), meta.kv_lens.tolist())
+    assert_close(out, want, torch.bfloat16, f"decode route {shape}")
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_no_workspace_within_the_limit(gpu, dtype):
     """A shape that would run split, called with no workspace: one launch, as before."""
@@ -86,7 +101,7 @@ def test_infinite_values_stay_infinite(ops, gpu, heads, keys):
         assert torch.allclose(got[:, rest].float(), want[:, rest], rtol=2.0 ** -8, atol=1e-4)
 
 
-@pytest.mark.parametrize("shape", [((64, 8), 193), ((16, 8), 8), ((4, 4), 400)], ids=str)
+@pytest.mark.parametrize("shape", [((64, 8), 100), ((16, 8), 8), ((32, 8), 200)], ids=str)
 def test_captured_call_within_the_limit_holds_no_workspace(ops, gpu, shape):
     """f32 shapes that run split within 1024 keys: captured in a graph they are one launch (the routes sum in
     different orders, so equal bits tell which one ran), and replays still match after the stream's workspace
