@@ -17,14 +17,34 @@ class _NoNative:
         return lambda *args: None
 
 
-def _both(monkeypatch, call):
+class _Recorder:
+    """The native module, noting which entry took a call (returned a tensor) and which declined."""
+
+    def __init__(self, native):
+        self.native, self.took, self.declined = native, [], []
+
+    def __getattr__(self, name):
+        def call(*args):
+            out = getattr(self.native, name)(*args)
+            (self.declined if out is None else self.took).append(name)
+            return out
+
+        return call
+
+
+def _both(monkeypatch, call, entry):
+    """The Python path first (it makes the stream's workspace), then the native one, which has to take the call."""
     from femtovllm import _C
 
-    got = call()
     with monkeypatch.context() as m:
         m.setattr(_C, "_native", _NoNative())
         want = call()
+    recorder = _Recorder(_C._native)
+    with monkeypatch.context() as m:
+        m.setattr(_C, "_native", recorder)
+        got = call()
     torch.cuda.synchronize()
+    assert recorder.took == [entry] and not recorder.declined
     assert got.shape == want.shape and got.stride() == want.stride() and got.dtype == want.dtype
     assert torch.equal(got.nan_to_num(nan=7.0), want.nan_to_num(nan=7.0))
     return got
@@ -51,7 +71,7 @@ def test_decode(ops, gpu, monkeypatch, dtype, dim, lens):
             wide = torch.full((tables.size(0), tables.size(1) + 5), -1, dtype=torch.int32, device=gpu)
             wide[:, : tables.size(1)] = tables
             tables = wide[:, : tables.size(1)]
-        _both(monkeypatch, lambda: ops.paged_attention_gemv(qf, wd.k_pool, wd.v_pool, tables, meta.kv_lens, meta.max_kv_len))
+        _both(monkeypatch, lambda: ops.paged_attention_gemv(qf, wd.k_pool, wd.v_pool, tables, meta.kv_lens, meta.max_kv_len), "gemv")
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
@@ -63,7 +83,7 @@ def test_prefill(ops, gpu, monkeypatch, dtype, dim):
     for qf in _forms(q.to(gpu)).values():
         _both(monkeypatch, lambda: ops.paged_attention_gemm(
             qf, wd.k_pool, wd.v_pool, meta.cu_seqlens, meta.max_q_len, meta.Q_TILE_SIZE, meta.cu_q_tiles,
-            meta.q_tile_to_seq_idx, meta.block_tables, meta.kv_lens, meta.positions))
+            meta.q_tile_to_seq_idx, meta.block_tables, meta.kv_lens, meta.positions), "gemm")
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
@@ -89,7 +109,42 @@ def test_prologue(ops, gpu, monkeypatch, dtype, packed, given):
         assert out is None or r is out
         return torch.cat([r.reshape(-1), kp.reshape(-1), vp.reshape(-1)])
 
-    _both(monkeypatch, call)
+    _both(monkeypatch, call, "prologue")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape", [(1, 4, 2, 70, 200), (2, 8, 8, 1, 33), (3, 6, 2, 129, 1)], ids=str)
+def test_dense(gpu, monkeypatch, dtype, shape):
+    from femtovllm import _C
+
+    B, H, KVH, Tq, Tk = shape
+    g = torch.Generator().manual_seed(4)
+    q, k, v = (torch.randn(s, generator=g).to(dtype).to(gpu) for s in ((B, H, Tq, 128), (B, KVH, Tk, 128), (B, KVH, Tk, 128)))
+    _both(monkeypatch, lambda: _C.FlashAttentionWarpCuda(q, k, v), "flash")
+
+
+def test_forms_left_to_the_python_path(ops, gpu, monkeypatch):
+    """A first call on a stream (no workspace yet), a subclass and a float max_kv_len: declined, the same result."""
+    from femtovllm import _C
+
+    class Sub(torch.Tensor):
+        pass
+
+    w = workloads.make_paged_workload("declined", [(1499, 1), (20, 1)], 4, 2, seed=55)
+    q, meta = w.gemv_call(device=gpu)
+    wd, q = w.to(gpu), q.to(gpu)
+    call = lambda q=q, n=meta.max_kv_len: ops.paged_attention_gemv(q, wd.k_pool, wd.v_pool, meta.block_tables, meta.kv_lens, n)
+    want = call()
+    torch.cuda.synchronize()
+    recorder = _Recorder(_C._native)
+    monkeypatch.setattr(_C, "_native", recorder)
+    with torch.cuda.stream(torch.cuda.Stream()):
+        _C._workspaces.pop((gpu.index, torch.cuda.current_stream(gpu).cuda_stream), None)
+        first = call()
+        torch.cuda.synchronize()
+    for got in (first, call(q=q.as_subclass(Sub)), call(n=float(meta.max_kv_len))):
+        assert torch.equal(got, want)
+    assert recorder.declined == ["gemv"] * 3 and not recorder.took
 
 
 def test_refused_calls_keep_their_errors(ops, gpu):
