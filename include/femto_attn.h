@@ -50,7 +50,8 @@ int femto_attn_kv_len_per_page(void);
 int femto_attn_dim_head(void);
 
 /* Bytes of workspace femto_paged_attention_gemv needs for these sizes when
- * it runs split (max_kv_len above the one-launch limit below).  It holds the
+ * it runs split (max_kv_len above the one-launch limit below, and some shapes
+ * within it, see there: without a workspace those run as one launch).  It holds the
  * per-split partial softmax states between the split kernel and the merge
  * kernel of one call; no initialisation is needed.  Calls that may overlap
  * (other streams) must not share a workspace. */
@@ -59,10 +60,10 @@ size_t femto_paged_attention_gemv_workspace_size(int num_seqs, int n_heads, int 
 /* Decode calls with max_kv_len at most this limit (default 1024 keys) run as
  * one kernel launch (a workgroup per sequence and KV head group) and use no
  * workspace; longer ones run the split kernel and the merge kernel.  At the
- * default, shapes that run faster split whatever the lengths (large batches
- * with eight query heads per KV head or in f32, and a few f32 sequences near
- * the limit) do so where a workspace is given, except under graph capture: a
- * captured call within the limit holds no workspace.  Sets the limit for the
+ * default, shapes that run faster split whatever the lengths (from four KV
+ * heads up, large batches with eight query heads per KV head, in f32 four; a
+ * few f32 sequences near the limit) do so where a workspace is given, except
+ * under graph capture: a captured call within the limit holds no workspace.  Sets the limit for the
  * process (-1: always split) and returns the previous one.
  * No counterpart in the reference (whose decode is always one launch,
  * csrc/paged_attention/paged_attention_gemv.cu:280-300); it exists for tests
@@ -76,7 +77,9 @@ int femto_attn_set_decode_single_max_kv(int max_kv_len);
  * called by femtovllm.ops.paged_attention_gemv (femtovllm/ops/__init__.py:82-107).
  * dtype: F32, F16 or BF16.  head_dim <= 128 (the reference's TORCH_CHECK_LE,
  * paged_attention_gemv.cu:256-257) in whole 16-byte chunks; scale 1/sqrt(head_dim).
- * kv_len == 0 yields a zero row, as in the reference.
+ * kv_len == 0 yields a zero row, as in the reference.  Rows of V past kv_len in
+ * the last page are not read; the last visible row stands for them with weight 0,
+ * so an infinity in it gives NaN, not an infinity, when kv_len is no multiple of 16.
  * workspace may be NULL (0 bytes) when max_kv_len is within the one-launch
  * limit of femto_attn_set_decode_single_max_kv. */
 int femto_paged_attention_gemv(

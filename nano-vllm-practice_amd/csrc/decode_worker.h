@@ -396,8 +396,12 @@ __device__ __forceinline__ void decode_segment(const DecodeArgs& a, int b, int k
         }
     };
 
-    // Three pages in flight: pages i+1 and i+2 load while page i
-    // computes (96 KB of loads per CU at one wave per SIMD).
+    // Registers of three pages, a page's loads issued two pages ahead.  Its
+    // block id is a pending load to the compiler wherever fetch_table may have
+    // run, so every issue waits out the loads before it: in effect the last
+    // page issued is in flight (32 KB per CU at one wave per SIMD) while the
+    // others are computed.  Exact waits, with three pages really in flight,
+    // ran 64 sequences of 256-4096 keys 5 % slower.
     PageRegs<E> r0, r1, r2;
     bool k0 = false, k1 = false, k2 = false;
     fetch_table(0);

@@ -495,6 +495,9 @@ int femto_paged_attention_gemm(int dtype, const void* q, int64_t q_stride_head, 
             // 1 / 16 / 31 rows on 8 KV heads 40.5 -> 38.5, 65.3 -> 57.8,
             // 72.9 -> 68.8 us; 4 uneven chunks without rows 51.5 -> 50.1 us;
             // 48 rows 93.6 -> 94.0 and, beside 64 tokens, 44.5 -> 45.2 us.
+            // (Few rows of equal contexts, cut alike, all end with the fold: 4
+            // of 2000 keys beside 64 tokens 16.6 -> 17.3 us, with lengths
+            // spread over a factor of eight 15 % faster.)
             // Groups of four heads keep the merge launch: the fold costs the
             // tiles' kernel its registers (256, and 2x slower workers).
             const int group = femto::prefill_group(a.n_rep);

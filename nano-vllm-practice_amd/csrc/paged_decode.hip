@@ -16,8 +16,8 @@
 //    non-temporal hint (each byte is read once per call), and the q.k
 //    reduction stays inside a DPP row;
 //  * block ids are fetched 64 at a time (one per lane) and broadcast with
-//    readlane, and each wave keeps three pages of loads in flight, so the
-//    table never adds a dependent load per page;
+//    readlane, and a page's loads go out two pages ahead of its math, so
+//    the table never adds a dependent load per page;
 //  * every lane keeps an online-softmax state (max, sum, 8 accumulators) per
 //    query head over the keys it saw; states merge across the four DPP rows
 //    with permlane swaps, each sequence segment of a slice leaves one partial
@@ -27,7 +27,8 @@
 //  * rows past kv_len are never read (loads are clamped to the last visible
 //    row and their scores masked) and block ids outside the pool are never
 //    dereferenced (their page reads as zeros), so NaN in unused pool memory
-//    cannot leak.
+//    cannot leak.  The repeated row has weight 0: where it holds an infinity
+//    of V, that output is NaN and not infinite.
 #include "decode_worker.h"
 
 namespace femto {
@@ -41,11 +42,11 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(DecodeArgs a) {
 // (sequence, KV head group), wave w taking the w-th of W contiguous shares
 // of the sequence's pages; the waves fold their states through LDS and
 // write the normalised rows, so no workspace and no merge launch are needed.
-// Decode calls only (query row b, kv_lens[b] keys).  W = 8 in calls of at most
-// one workgroup per CU, whose waves then walk half as many pages (the chain of
-// page loads and page math of a wave sets the length of such a call), else 4:
-// eight-wave workgroups would take more rounds (64 sequences of up to 512 keys
-// on 16/8 heads 18.6 us with four waves, 21.6 with eight).  decode_route picks.
+// Decode calls only (query row b, kv_lens[b] keys).  W = 8 lets each wave walk
+// half as many pages, whose chain of loads and math sets the length of a call
+// of one workgroup per CU; with more workgroups than CUs it takes more rounds
+// (64 sequences of up to 512 keys on 16/8 heads 18.6 us with four waves, 21.6
+// with eight).  decode_route picks.
 template <typename E, int NREP, bool FULL, int W>
 __global__ __launch_bounds__(64 * W) void paged_decode_single_kernel(DecodeArgs a) {
     __shared__ float s_ml[W][NREP][2];
@@ -167,8 +168,8 @@ __global__ __launch_bounds__(128) void paged_decode_merge_kernel(DecodeArgs a) {
     if (t < a.head_dim) store_elem<E>(out, o, O / L);
 }
 
-// One wave per SIMD (4 per CU), each with three pages of K and V in flight
-// (96 KB per CU).  HBM read throughput peaks there: more resident waves queue
+// One wave per SIMD (4 per CU), each with a page of K and V in flight behind
+// those it computes.  HBM read throughput peaks there: more resident waves queue
 // more requests and lose bandwidth (on the 545 MB Qwen3-0.6B-shaped batch, 16
 // waves per CU ran at 4.85 TB/s and 4 per CU at 5.2 TB/s with ordinary loads;
 // 8 per CU with non-temporal loads was 2 % slower than 4, and 6 or 8 per CU

@@ -36,8 +36,11 @@
 //    enough (every P is at most its growth): more than kMaxBlockSum, or
 //    infinite, and the block's maximum is taken and its exponentials are
 //    redone before P.V reads them.  The first tile has no running max and
-//    takes its maximum over both blocks.  Inputs with a tile-by-tile rising maximum take that
-//    path once per growth of the sum past 2^8.  Against a maximum per tile
+//    takes its maximum over both blocks.  Sharp scores, whose maxima
+//    keep growing past 2^8, take that path on many of a row's first tiles:
+//    8 x 512 on 16/8 heads 87.2 -> 92.3 us with scores spread over ~12 log2
+//    units, 82.4 -> 96.0 over ~90 (80.3 against 82.7 at 1.4, 87.0 against 85.7
+//    at 6).  Against a maximum per tile
 //    before the first exponential: 2048 x 8192 dense 252 -> 240 us, the last
 //    2048 tokens of a 32k prompt 963 -> 955 us, 8 x 512 73.3 -> 72.6 us, 4
 //    uneven sequences 51.9 -> 51.0 us (MFMA busy 56 -> 63 % dense, 59 -> 60 %
